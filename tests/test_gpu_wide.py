@@ -1,0 +1,52 @@
+"""Ray batches over the device-built 4-wide tree against the counting kernel, which walks the
+reference's rows: the same primitives and distance bits; any-hits against the host build of
+the rows' walk.  Scenes the wide tree refuses (a caller's boxes that are not the triangles'
+own, trees deeper than its builder goes) render over the rows."""
+import numpy as np
+import pytest
+
+from tests import wide_rays
+from zillumgl_amd import render, scene
+
+pytestmark = pytest.mark.gpu
+SCENES = wide_rays.scenes()
+
+
+@pytest.fixture(scope="module")
+def probe(tmp_path_factory):
+    return wide_rays.Probe(tmp_path_factory.mktemp("wide"))
+
+
+def _compare(probe, ps, n):
+    r = wide_rays.rays(ps, n)
+    ctx = render.Context(0)
+    try:
+        ctx.upload(ps)
+        prim, t, b = ctx.trace_closest(r)
+        ref = ctx.trace_closest(r, counted=True)
+        np.testing.assert_array_equal(prim, ref[0])
+        np.testing.assert_array_equal(t.view(np.int32), ref[1].view(np.int32))
+        np.testing.assert_array_equal(b, ref[2])
+        tm = wide_rays.limits(ps, n)
+        probe.build(ps)
+        want, _, _ = probe.trace(r, tm, rows_only=True)
+        np.testing.assert_array_equal(ctx.trace_any(r, tm), want >= 0)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("name", sorted(SCENES))
+def test_batches_equal_the_rows(probe, name):
+    _compare(probe, scene.pack(SCENES[name]), 20000)
+
+
+@pytest.mark.parametrize("n", [1000, 100003])
+def test_batch_sizes(probe, n):
+    ps = scene.pack(scene.config5(32, 32, n=20, env_size=(8, 4)))  # above the rule's 2,048 triangles
+    _compare(probe, ps, n)
+
+
+def test_boxes_larger_than_their_triangles(probe):
+    ps = scene.pack(scene.config5(32, 32, n=20, env_size=(8, 4)))
+    ps.bounds = (ps.bounds + np.array([-1, -1, -1, 1, 1, 1], np.float32) * np.float32(0.05)).astype(np.float32)
+    _compare(probe, ps, 5000)

@@ -153,7 +153,9 @@ ZGL_D double remZ(const Sum3& a) { return a.z + a.ez; }
 // first pass records every closest-hit query (primitive, distance) and every shadow
 // query (occluded) in order, and the replay pass reads them back.  Either way the queries
 // are the same, with the same rays, as the walks that produced the log, so are the
-// results.  Queries past the log's capacity (paths deeper than the log holds) are walked.
+// results.  Queries past the log's capacity (paths deeper than the log holds) are walked
+// over the rows: the wide walk's registers and stack would cost the kernel, which hardly
+// ever walks, a wave per SIMD (253 VGPRs against 236).
 constexpr int kHitLog = kHitLogQueries;
 struct HitLog {
     int n;
@@ -173,8 +175,8 @@ template <bool ADJ> ZGL_D int loggedHit(const DevScene& s, const Ray& r, float& 
         dist = log.dist[i];
         return log.id[i];
     }
-    Counters cn;
-    const int id = bvhHit<false>(s, r, dist, cn);
+    dist = 1e8f;
+    const int id = walkRowsOnly<false>(s, r, dist);
     if (!ADJ && i < kHitLog) {
         log.id[i] = id;
         log.dist[i] = dist;
@@ -186,8 +188,7 @@ template <bool ADJ> ZGL_D bool loggedTest(const DevScene& s, const Ray& r, float
     const int i = log.n++;
     if (log.pre && i < kHitLog) return log.pre[i].x != 0;
     if (ADJ && i < kHitLog) return log.id[i] != 0;
-    Counters cn;
-    const bool occluded = bvhTest<false>(s, r, tmax, cn);
+    const bool occluded = walkRowsOnly<true>(s, r, tmax) >= 0;
     if (!ADJ && i < kHitLog) log.id[i] = occluded ? 1 : 0;
     return occluded;
 }

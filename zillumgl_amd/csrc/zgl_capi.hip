@@ -149,6 +149,7 @@ struct zgl_context {
     // differentiable mode: evaluation point, adjoint input and outputs
     DevBuf evalMat, evalEnv, dFrame, dMat, dEnv;
     DevBuf bvhBounds;  // node bounds of a device-built MTBVH
+    DevBuf wide;       // 4-wide tree, then its builder's work memory
     DevBuf gqQueues, gqCounts;  // global-queue path tracer
     int gqBlocksPerCU = 0;
     DevBuf wfWork;    // wavefront schedule of the naive tracer
@@ -182,7 +183,7 @@ struct zgl_context {
                          &lightPower, &lightAlias, &lightProb, &env, &envAlias, &envProb, &noise, &sobolM,
                          &sobolTab, &frame, &film, &counters, &scratchRays, &scratchOut, &workCounter,
                          &evalMat, &evalEnv, &dFrame, &dMat, &dEnv, &bvhBounds, &gqQueues, &gqCounts, &wfWork,
-                         &naiveRes, &hitLog, &refSum, &tex, &texScale, &texRaw};
+                         &naiveRes, &hitLog, &refSum, &tex, &texScale, &texRaw, &wide};
         for (DevBuf* b : all) b->release();
         bvh.release();
     }
@@ -476,6 +477,21 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
                                           ctx->stream, msg);
             if (rc) throw ZglError{rc == 1 ? ZGL_E_INVALID : (rc == 3 ? ZGL_E_OOM : ZGL_E_HIP), msg};
         }
+        // a device too full for the wide tree renders over the rows, with the same results
+        WideScale wideScale{};
+        const size_t wideBytes = (size_t)wideCapacity(nT) * 64;
+        bool wideFits = true;
+        try {
+            ctx->ensure(ctx->wide, wideBytes + wideWorkBytes(nT), "wide tree");
+        } catch (const ZglError& e) {
+            if (e.code != ZGL_E_OOM) throw;
+            (void)hipGetLastError();
+            wideFits = false;
+        }
+        if (wideFits)
+            hipCheck(buildWide((const float4*)ctx->rows.p, (const float4*)ctx->tris.p, nT,
+                               (char*)ctx->wide.p + wideBytes, (uint4*)ctx->wide.p, ctx->stream, wideScale),
+                     "wide tree build");
         ctx->upload(ctx->normals, sb->normals, (size_t)nV * 12, "normals");
         ctx->upload(ctx->texcoords, sb->texcoords, (size_t)sb->n_texcoords * 8, "texcoords");
         ctx->upload(ctx->matTex, sb->mat_tex_indices, (size_t)sb->obj_prim_count * 4, "matTexIndices");
@@ -492,6 +508,10 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
         DevScene& s = ctx->scene;
         s.rows = (const float4*)ctx->rows.p;
         s.tris = (const float4*)ctx->tris.p;
+        s.wide = wideScale.ok ? (const uint4*)ctx->wide.p : nullptr;
+        s.wideUnit = wideScale.unit;
+        s.wideSlack = 4.0f * wideScale.pad;
+        s.wideBound = wideScale.bound;
         s.indices = (const int32_t*)ctx->indices.p;
         s.vertices = (const float*)ctx->vertices.p;
         s.normals = (const float*)ctx->normals.p;

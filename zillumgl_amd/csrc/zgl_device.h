@@ -17,6 +17,7 @@
 
 #include "zgl_box.h"
 #include "zgl_math.h"
+#include "zgl_wide.h"
 
 namespace zgl {
 
@@ -39,6 +40,8 @@ constexpr int SobolSampleDim = 256;
 struct DevScene {
     const float4* rows;          // 6 * bvhSize * 2
     const float4* tris;          // nTriangles * 3
+    const uint4* wide;           // 4-wide tree of the same leaves (zgl_wide.h), or null
+    float wideUnit, wideSlack, wideBound;
     const int32_t* indices;      // 3 per triangle
     const float* vertices;       // 3 per vertex
     const float* normals;        // 3 per vertex
@@ -103,26 +106,43 @@ struct Counters {
 };
 template <bool C> ZGL_D void cnt(Counters& c, uint32_t b) { if (C) c.bytes += b; }
 
-// The row table and the triangle positions as seen by a walk loop: loaded from the
-// scene once before the loop and held in scalar registers.  Read through the scene at
-// every step, the compiler reloads the pointer from the kernel arguments inside each
-// row step, which puts a scalar load and its wait on every row's dependent chain; the
-// empty asm keeps it from doing so.  The pointers keep the global address space, so the
-// loads stay global loads.
-typedef float GFloat4 __attribute__((ext_vector_type(4)));
-typedef const GFloat4 __attribute__((address_space(1)))* GRows;
-typedef const float __attribute__((address_space(1)))* GFloats;
-struct WalkMem {
-    GRows rows;
-    GRows tris;
-};
-ZGL_D WalkMem walkMem(const DevScene& s)
+// The scene's walk data as seen by a walk loop: loaded from the scene once before the loop
+// and held in scalar registers.  Read through the scene at every step, the compiler
+// reloads the pointers from the kernel arguments inside each step, which puts a scalar
+// load and its wait on every step's dependent chain; the empty asm keeps it from doing
+// so.  The pointers keep the global address space, so the loads stay global loads.
+// The byte-counting variants (C) count the reference's rows and take no other.
+template <bool C> ZGL_D WalkMem walkMem(const DevScene& s)
 {
-    WalkMem m{(GRows)s.rows, (GRows)s.tris};
+    WalkMem m{(GRows)s.rows, (GRows)s.tris, C ? (WideSlots) nullptr : (WideSlots)s.wide, s.bvhSize, s.wideUnit,
+              s.wideSlack, s.wideBound};
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+s"(m.rows), "+s"(m.tris));
+    asm volatile("" : "+s"(m.rows), "+s"(m.tris), "+s"(m.wide));
 #endif
     return m;
+}
+
+// The walk stacks of a workgroup of at most kWalkLanes lanes in one dimension: entry i of a
+// lane lies kWalkLanes words after entry i - 1, child words and keys apart, so that the
+// lanes of a wave reach different banks whatever their depths.
+struct LdsStack {
+    uint32_t* base;
+    ZGL_D WalkEntry get(int i) const
+    {
+        const uint32_t* e = base + i * (2 * kWalkLanes);
+        return WalkEntry{e[0], e[kWalkLanes]};
+    }
+    ZGL_D void put(int i, WalkEntry x) const
+    {
+        uint32_t* e = base + i * (2 * kWalkLanes);
+        e[0] = x.word;
+        e[kWalkLanes] = x.key;
+    }
+};
+ZGL_D LdsStack walkStack()
+{
+    __shared__ uint32_t mem[2 * kWalkStack * kWalkLanes];
+    return LdsStack{mem + threadIdx.x};
 }
 
 // ---------------------------------------------------------------------------
@@ -172,7 +192,60 @@ ZGL_D void envRotCSN(const DevScene& s, double& c, double& sn) { sincosF64(-(dou
 // the rendering path's instance of the library (made zgl's by the using-directive of
 // zgl_math.h)
 namespace f32 {
+// One round of a walk: kNodes steps over the wide tree, then the triangle put by; or four
+// of the reference's rows.  The lanes of a wave come to triangles at different steps:
+// putting one by and going on keeps their lanes busy, and testing once per round keeps
+// the triangle test from running on nearly every step for a few lanes.  Returns true when
+// the walk has ended.  If it then is kWalkPending, walkSettle has to settle it before its
+// result is used; a walk that found nothing is not.
+template <bool C, int kNodes> ZGL_D bool walkRound(const WalkMem& m, Walk& w, LdsStack& st, Counters& cn)
+{
+    bool done = false;
+    if (!C && !(w.flags & kWalkRows)) {
+#pragma unroll
+        for (int u = 0; u < kNodes; u++) wideStep(m, w, st);
+        if (w.leaf >= 0) done = wideLeaf(m, w);
+        done = done || (w.cur == kWalkNone && w.sp == 0);
+        if (done && w.closest != -1) w.flags |= kWalkPending;
+    } else {
+        uint32_t rows = 0, tests = 0;
+        done = rowsStep(m, w, __ballot(!generalRay(w)) == 0ull, rows, tests);
+        if (C) {
+            cn.rows += rows;
+            cn.tests += tests;
+            cn.bytes += 36 * rows + 48 * tests;
+        }
+    }
+    return done;
+}
+// Settles a walk that ended kWalkPending; false when it goes on, over the rows.  The
+// resumable schedules walk those rays among the others, with the wave's next rounds; a
+// walk by one lane (CHAIN) would hold up its wave for a hundred rows and asks the hit's
+// ancestors first.
+template <bool CHAIN> ZGL_D bool walkSettle(const WalkMem& m, Walk& w)
+{
+    w.flags &= ~kWalkPending;
+    if (wideSettle<CHAIN>(m, w)) return true;
+    walkRows(m, w);
+    return false;
+}
+// A whole walk by one lane: the closest hit's primitive (dist 1e8 on a miss), or any.
+ZGL_D int walkAll(const DevScene& s, vec3 o, vec3 d, bool any, float& dist)
+{
+    const WalkMem m = walkMem<false>(s);
+    Counters cn;
+    LdsStack st = walkStack();
+    Walk w;
+    walkStart(m, w, o, d, any, dist);
+    do {
+        while (!walkRound<false, 1>(m, w, st, cn)) {}
+    } while ((w.flags & kWalkPending) && !walkSettle<true>(m, w));
+    dist = w.dist;
+    return w.closest;
+}
+#define ZGL_WIDE_WALK 1
 #include "zgl_device_body.inc"
+#undef ZGL_WIDE_WALK
 }  // namespace f32
 
 // Film splat of the light-path integrators (light_path_integ.glsl:34-43, addImage); the

@@ -42,6 +42,13 @@ struct BatchScene {
     int threshold;  // lanes still walking when a wave working on this scene stops to shade
 };
 
+// The 4-wide tree of a scene's rows and triangles (zgl_wide.hip): slots holds
+// wideCapacity(n) slots of 64 bytes, work wideWorkBytes(n) bytes.  scale.ok is false where
+// the scene has no wide tree (its rays then take the rows).  Synchronises the stream.
+int64_t wideCapacity(int64_t nTri);
+size_t wideWorkBytes(int64_t nTri);
+hipError_t buildWide(const float4* rows, const float4* tris, int64_t nTri, void* work, uint4* slots, hipStream_t st,
+                     WideScale& scale);
 hipError_t launchSobolTable(const uint32_t* sobolM, uint32_t* tab, int first, int count, hipStream_t st);
 hipError_t launchFill(float* p, int64_t n, float v, hipStream_t st);
 hipError_t launchSrgbExpand(const uint8_t* rgb, const float* lut, float4* out, int64_t n, hipStream_t st);

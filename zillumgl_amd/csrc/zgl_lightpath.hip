@@ -38,7 +38,7 @@ enum : int {
     kDone,
 };
 
-constexpr int kRowsPerRound = 4;
+constexpr int kNodesPerRound = 3;  // as the naive tracer's
 
 __global__ void k_reset_light_counter(int* c) { if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0; }
 
@@ -63,9 +63,8 @@ __global__ __launch_bounds__(256, 4) void k_lightpath_persistent(DevScene s0, Pa
     int loopsLeft = 0;
     bool walking = false;
     Walk wk;
-    wk.p.o = v3(0.f); wk.p.d = v3(0.f); wk.p.dInv = v3(0.f); wk.p.mode = 0;
-    wk.p.nx = wk.p.ny = wk.p.nz = false; wk.p.table = 0;
-    wk.dist = 0.f; wk.k = 0; wk.closest = -1; wk.any = false;
+    walkIdle(wk);
+    LdsStack stack = walkStack();
     Rng rng = {0u, 0u, 0, 0};
     vec3 throughput = v3(0.f), wo = v3(0.f);
     Ray next = makeRay(v3(0.f), v3(0.f));  // the extension ray issued after the connection
@@ -80,12 +79,13 @@ __global__ __launch_bounds__(256, 4) void k_lightpath_persistent(DevScene s0, Pa
 
     for (;;) {
         const DevScene& s = sceneArg(s0);
+        const WalkMem wm = walkMem<false>(s);
         auto endPath = [&]() { phase = loopsLeft > 0 ? kStart : kNewUnit; };
         // after a connection walk: the splat if unoccluded, then the extension walk or the end
         auto settle = [&]() {
             if (wk.closest < 0 && pendValid) splatFilm(s, film, pendUv, pendRes);
             if (cont) {
-                walkStart<false>(s, wk, next, false, 1e8f, cn);
+                walkStart<false>(wm, wk, next, false, 1e8f, cn);
                 walking = true;
                 phase = kExtend;
             } else {
@@ -95,11 +95,11 @@ __global__ __launch_bounds__(256, 4) void k_lightpath_persistent(DevScene s0, Pa
         // the walk a state ends with: the connection if there is one, else the extension
         auto issue = [&](bool connect, const Ray& vis, float visDist) {
             if (connect) {
-                walkStart<false>(s, wk, vis, true, visDist, cn);
+                walkStart<false>(wm, wk, vis, true, visDist, cn);
                 walking = true;
                 phase = kConnect;
             } else if (cont) {
-                walkStart<false>(s, wk, next, false, 1e8f, cn);
+                walkStart<false>(wm, wk, next, false, 1e8f, cn);
                 walking = true;
                 phase = kExtend;
             } else {
@@ -150,6 +150,7 @@ __global__ __launch_bounds__(256, 4) void k_lightpath_persistent(DevScene s0, Pa
             issue(connect, vis, visDist);
         };
 
+        if (!walking && (wk.flags & kWalkPending)) walking = !walkSettle<false>(wm, wk);
         if (!walking) {
             if (phase == kConnect) {
                 settle();
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(256, 4) void k_lightpath_persistent(DevScene s0, Pa
                     endPath();
                 } else {
                     const float dist = wk.dist;
-                    const vec3 pos = rayPoint(makeRay(wk.p.o, wk.p.d), dist);
+                    const vec3 pos = rayPoint(makeRay(wk.o, wk.d), dist);
                     SurfaceInfo surf = triangleSurfaceInfo<false>(s, id, pos, cn);
                     const int matTex = s.matTexIndices[id];
                     const int matId = matTex & 0x0000ffff;
@@ -265,22 +266,11 @@ __global__ __launch_bounds__(256, 4) void k_lightpath_persistent(DevScene s0, Pa
         while (!walking && phase == kStart) startPath();
         if (__ballot(phase != kDone) == 0ull) break;
 
-        // walking: up to kRowsPerRound rows per lane per round, leaves tested together once
-        // per round; a finished connection walk splats and starts its extension walk here
-        bool general = __ballot(walking && wk.p.special) == 0ull;
-        const WalkMem wm = walkMem(s);
+        // walking, a round at a time; a finished connection walk splats and starts its
+        // extension walk here
         for (;;) {
-#pragma unroll
-            for (int u = 0; u < kRowsPerRound; ++u) {
-                if (walking && wk.leaf < 0) {
-                    if (walkRow<false>(wm, wk, general, cn)) walking = false;
-                }
-            }
-            if (walking && wk.leaf >= 0) {
-                if (walkLeaf<false>(wm, wk, cn)) walking = false;
-            }
-            if (!walking && phase == kConnect) settle();
-            general = __ballot(walking && wk.p.special) == 0ull;
+            if (walking && walkRound<false, kNodesPerRound>(wm, wk, stack, cn)) walking = false;
+            if (!walking && phase == kConnect && !(wk.flags & kWalkPending)) settle();
             if (__popcll(__ballot(walking)) <= threshold) break;
         }
     }

@@ -4,8 +4,8 @@
 //   * every lane owns one pixel at a time and renders that pixel's passes in order,
 //     so its running sum is formed exactly as one launch per pass would form it;
 //   * a lane's path is a state machine whose states end by issuing one ray (camera,
-//     shadow or extension).  Walks advance one MTBVH row per step for all lanes of the
-//     wave; when a ballot shows that no more than `threshold` lanes are still walking,
+//     shadow or extension).  Walks (zgl_wide.h) advance a round at a time for all lanes
+//     of the wave; when a ballot shows that no more than `threshold` lanes are still walking,
 //     the lanes whose walk finished run their shading transition and issue their next
 //     ray, so lanes with short walks do not wait for the longest walk of the wave;
 //   * lanes that finish all passes of their pixel take the next pixel from a global
@@ -34,9 +34,11 @@ enum : int {
     kWait,      // batch: the wave's scene has no pixels left; wait for the next scene
 };
 
-// MTBVH rows each walking lane advances per round of the walking loop (one leaf test
-// and one ballot per round).
-constexpr int kRowsPerRound = 4;
+// Nodes of the wide tree each walking lane advances per round of the walking loop (one
+// triangle test and one ballot per round).  1 / 2 / 3 / 4: 124.0 / 116.5 / 114.8 / 114.9 ms
+// on the headline launch, 24.5 / 23.0 / 22.3 / 21.9 ms on ten batched scenes, 2.78 / 2.69 /
+// 2.70 / 2.80 ms on the material scene.
+constexpr int kNodesPerRound = 3;
 constexpr int kRegions = kUnitRegions;  // unit regions, one per XCD
 
 // Pixel order for the dynamic fetch: 8x8 tiles in row-major tile order.
@@ -101,9 +103,8 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
     uint32_t pendBytes = 0;
     bool walking = false;
     Walk wk;
-    wk.p.o = v3(0.f); wk.p.d = v3(0.f); wk.p.dInv = v3(0.f); wk.p.mode = 0;
-    wk.p.nx = wk.p.ny = wk.p.nz = false; wk.p.table = 0;
-    wk.dist = 0.f; wk.k = 0; wk.closest = -1; wk.any = false;
+    walkIdle(wk);
+    LdsStack stack = walkStack();
 
     for (;;) {
         const int csu = BATCH ? __builtin_amdgcn_readfirstlane(cs) : 0;
@@ -130,13 +131,16 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
             }
         };
 
+        const WalkMem wm = walkMem<C>(s);
+
         // ------------------------------------------------------------ shading
+        if (!walking && (wk.flags & kWalkPending)) walking = !walkSettle<false>(wm, wk);
         if (!walking) {
             // completion of the ray that was walked
             if (phase == kPrimary) {
                 logQuery(false);
                 const int id = wk.closest;
-                const Ray ray = makeRay(wk.p.o, wk.p.d);
+                const Ray ray = makeRay(wk.o, wk.d);
                 pos = rayPoint(ray, wk.dist);
                 if (id == -1) {
                     result = envLe<C>(s, ray.dir, cn);
@@ -159,7 +163,7 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
                 }
                 if (terminate) phase = kFinish;
                 else {
-                    walkStart<C>(s, wk, rayOffseted(pos, wi), false, 1e8f, cn);
+                    walkStart<C>(wm, wk, rayOffseted(pos, wi), false, 1e8f, cn);
                     walking = true;
                     phase = kExtend;
                 }
@@ -167,7 +171,7 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
                 logQuery(false);
                 const int nextId = wk.closest;
                 const int lightId = nextId - s.objPrimCount;
-                const vec3 nextPos = rayPoint(makeRay(wk.p.o, wk.p.d), wk.dist);
+                const vec3 nextPos = rayPoint(makeRay(wk.o, wk.d), wk.dist);
                 if (nextId == -1) {
                     vec3 radiance = envLe<C>(s, wi, cn);
                     float weight = 1.0f;
@@ -290,13 +294,13 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
                     rrProb = fminG(maxComponent(bs.bsdf / bsdfPdf), 0.95f);
                 }
                 if (shadow) {
-                    walkStart<C>(s, wk, shadowRay, true, shadowDist, cn);
+                    walkStart<C>(wm, wk, shadowRay, true, shadowDist, cn);
                     walking = true;
                     phase = kShadow;
                 } else if (terminate) {
                     phase = kFinish;
                 } else {
-                    walkStart<C>(s, wk, rayOffseted(pos, wi), false, 1e8f, cn);
+                    walkStart<C>(wm, wk, rayOffseted(pos, wi), false, 1e8f, cn);
                     walking = true;
                     phase = kExtend;
                 }
@@ -365,7 +369,7 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
             query = 0;
             if (C) cn.bytes += 64 + 32;
             const vec4 u = sample4D<C>(s, rng, cn);
-            walkStart<C>(s, wk, cameraSampleRay(s, scr, u), false, 1e8f, cn);
+            walkStart<C>(wm, wk, cameraSampleRay(s, scr, u), false, 1e8f, cn);
             walking = true;
             phase = kPrimary;
         }
@@ -383,28 +387,15 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
         if (__ballot(phase != kDone) == 0ull) break;
 
         // ------------------------------------------------------------ walking
-        // Each round advances every walking lane by up to kRowsPerRound rows; a lane
-        // that reaches a leaf whose box is hit waits there, and the waiting lanes test
-        // their triangles together once per round, so that the triangle test (as long
-        // as the box test) runs once per round instead of on nearly every row step for
-        // a few lanes.  A lane whose shadow walk ends settles its NEE term and starts its
-        // extension walk within the loop (the same operations, in the same order, as the
-        // shading step would do), instead of idling until the wave leaves the loop.
+        // A lane whose shadow walk ends settles its NEE term and starts its extension walk
+        // within the loop (the same operations, in the same order, as the shading step
+        // would do), instead of idling until the wave leaves the loop; waiting for four or
+        // eight such lanes costs more than it saves (114.6 -> 116.8 / 120.3 ms).
         {
-            bool general = __ballot(walking && wk.p.special) == 0ull;
-            const WalkMem wm = walkMem(s);
             for (;;) {
-#pragma unroll
-                for (int u = 0; u < kRowsPerRound; ++u) {
-                    if (walking && wk.leaf < 0) {
-                        if (walkRow<C>(wm, wk, general, cn)) walking = false;
-                    }
-                }
-                if (walking && wk.leaf >= 0) {
-                    if (walkLeaf<C>(wm, wk, cn)) walking = false;
-                }
+                if (walking && walkRound<C, kNodesPerRound>(wm, wk, stack, cn)) walking = false;
                 // a shadow walk that ended settles its NEE term and starts the extension walk
-                if (!walking && phase == kShadow) {
+                if (!walking && phase == kShadow && !(wk.flags & kWalkPending)) {
                     logQuery(true);
                     if (wk.closest < 0) {
                         if (C) cn.bytes += pendBytes;
@@ -413,12 +404,11 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
                     if (terminate) {
                         phase = kFinish;
                     } else {
-                        walkStart<C>(s, wk, rayOffseted(pos, wi), false, 1e8f, cn);
+                        walkStart<C>(wm, wk, rayOffseted(pos, wi), false, 1e8f, cn);
                         walking = true;
                         phase = kExtend;
                     }
                 }
-                general = __ballot(walking && wk.p.special) == 0ull;
                 if (__popcll(__ballot(walking)) <= sceneThreshold) break;
             }
         }
@@ -511,16 +501,17 @@ __global__ __launch_bounds__(256, 4) void k_triple_persistent(DevScene s0, PassP
     vec3 pend = v3(0.f);
     bool walking = false;
     Walk wk;
-    wk.p.o = v3(0.f); wk.p.d = v3(0.f); wk.p.dInv = v3(0.f); wk.p.mode = 0;
-    wk.p.nx = wk.p.ny = wk.p.nz = false; wk.p.table = 0;
-    wk.dist = 0.f; wk.k = 0; wk.closest = -1; wk.any = false;
+    walkIdle(wk);
+    LdsStack stack = walkStack();
 
     for (;;) {
         const DevScene& s = sceneArg(s0);
+        const WalkMem wm = walkMem<false>(s);
+        if (!walking && (wk.flags & kWalkPending)) walking = !walkSettle<false>(wm, wk);
         if (!walking) {
             if (phase == kPrimary) {
                 const int hit = wk.closest;
-                const Ray ray = makeRay(wk.p.o, wk.p.d);
+                const Ray ray = makeRay(wk.o, wk.d);
                 const float primDist = wk.dist;
                 pos = rayPoint(ray, primDist);
                 if (hit == -1) {
@@ -549,14 +540,14 @@ __global__ __launch_bounds__(256, 4) void k_triple_persistent(DevScene s0, PassP
                 if (terminate) {
                     phase = kFinish;
                 } else {
-                    walkStart<false>(s, wk, rayOffseted(pos, wi), false, 1e8f, cn);
+                    walkStart<false>(wm, wk, rayOffseted(pos, wi), false, 1e8f, cn);
                     walking = true;
                     phase = kExtend;
                 }
             } else if (phase == kExtend) {
                 const int nextId = wk.closest;
                 const int lightId = nextId - s.objPrimCount;
-                const vec3 nextPos = rayPoint(makeRay(wk.p.o, wk.p.d), wk.dist);
+                const vec3 nextPos = rayPoint(makeRay(wk.o, wk.d), wk.dist);
                 const float dist = wk.dist;
                 if (nextId == -1) {
                     phase = kFinish;
@@ -649,13 +640,13 @@ __global__ __launch_bounds__(256, 4) void k_triple_persistent(DevScene s0, PassP
                     prevNorm = surf.ns;
                 }
                 if (shadow) {
-                    walkStart<false>(s, wk, shadowRay, true, shadowDist, cn);
+                    walkStart<false>(wm, wk, shadowRay, true, shadowDist, cn);
                     walking = true;
                     phase = kShadow;
                 } else if (terminate) {
                     phase = kFinish;
                 } else {
-                    walkStart<false>(s, wk, rayOffseted(pos, wi), false, 1e8f, cn);
+                    walkStart<false>(wm, wk, rayOffseted(pos, wi), false, 1e8f, cn);
                     walking = true;
                     phase = kExtend;
                 }
@@ -715,7 +706,7 @@ __global__ __launch_bounds__(256, 4) void k_triple_persistent(DevScene s0, PassP
             rng.sampleOffset = sampleOffsetOf(spp);
             rng.dim = 0;
             const vec4 u = sample4D<false>(s, rng, cn);
-            walkStart<false>(s, wk, cameraSampleRay(s, scr, u), false, 1e8f, cn);
+            walkStart<false>(wm, wk, cameraSampleRay(s, scr, u), false, 1e8f, cn);
             walking = true;
             phase = kPrimary;
         }
@@ -723,30 +714,19 @@ __global__ __launch_bounds__(256, 4) void k_triple_persistent(DevScene s0, PassP
         if (__ballot(phase != kDone) == 0ull) break;
 
         {
-            bool general = __ballot(walking && wk.p.special) == 0ull;
-            const WalkMem wm = walkMem(s);
             for (;;) {
-#pragma unroll
-                for (int u = 0; u < kRowsPerRound; ++u) {
-                    if (walking && wk.leaf < 0) {
-                        if (walkRow<false>(wm, wk, general, cn)) walking = false;
-                    }
-                }
-                if (walking && wk.leaf >= 0) {
-                    if (walkLeaf<false>(wm, wk, cn)) walking = false;
-                }
+                if (walking && walkRound<false, kNodesPerRound>(wm, wk, stack, cn)) walking = false;
                 // a visibility walk that ended settles its s=1 term and starts the extension
-                if (!walking && phase == kShadow) {
+                if (!walking && phase == kShadow && !(wk.flags & kWalkPending)) {
                     if (wk.closest < 0) result += pend;
                     if (terminate) {
                         phase = kFinish;
                     } else {
-                        walkStart<false>(s, wk, rayOffseted(pos, wi), false, 1e8f, cn);
+                        walkStart<false>(wm, wk, rayOffseted(pos, wi), false, 1e8f, cn);
                         walking = true;
                         phase = kExtend;
                     }
                 }
-                general = __ballot(walking && wk.p.special) == 0ull;
                 if (__popcll(__ballot(walking)) <= threshold) break;
             }
         }

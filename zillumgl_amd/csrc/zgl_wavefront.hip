@@ -29,7 +29,7 @@ namespace zgl {
 namespace {
 
 constexpr int kWfBlock = 256;
-constexpr int kWfRows = 4;      // MTBVH rows per walk round (as the persistent kernel)
+constexpr int kWfNodes = 2;     // nodes of the wide tree per walk round (as the persistent kernel)
 constexpr int kWfChunk = 256;   // rays a wave takes from the queue per atomic
 constexpr int kWfRefill = 8;    // idle lanes that make a wave take new rays
 
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kWfBlock) void k_wf_camera(DevScene s, int nIndex, 
 // ---------------------------------------------------------------- trace
 // Persistent walker: lanes take rays from the queue (a wave claims kWfChunk at a time)
 // whenever kWfRefill of them are idle or none walks, and walk them with the persistent
-// kernel's rounds (kWfRows rows, then one leaf test for the lanes at a leaf).
+// kernel's rounds (kWfNodes nodes, then one triangle test for the lanes at one).
 __global__ __launch_bounds__(kWfBlock) void k_wf_trace(DevScene s, const WfRay* __restrict__ rays,
                                                        const int* __restrict__ count, int* __restrict__ fetch,
                                                        WfState st)
@@ -173,9 +173,9 @@ __global__ __launch_bounds__(kWfBlock) void k_wf_trace(DevScene s, const WfRay* 
     const int lane = threadIdx.x & 63;
     Counters cn;
     Walk wk;
-    wk.p.o = v3(0.f); wk.p.d = v3(0.f); wk.p.dInv = v3(0.f); wk.p.mode = 0;
-    wk.p.nx = wk.p.ny = wk.p.nz = false; wk.p.special = false; wk.p.table = 0;
-    wk.dist = 0.f; wk.k = 0; wk.end = 0; wk.closest = -1; wk.leaf = -1; wk.any = false;
+    walkIdle(wk);
+    LdsStack stack = walkStack();
+    const WalkMem wm = walkMem<false>(s);
     bool walking = false;
     bool own = false;  // the lane holds a ray whose result is still to be stored
     int tag = 0;
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(kWfBlock) void k_wf_trace(DevScene s, const WfRay* 
                     Ray ray;
                     ray.ori = v3(r.oT.x, r.oT.y, r.oT.z);
                     ray.dir = v3(r.dP.x, r.dP.y, r.dP.z);
-                    walkStart<false>(s, wk, ray, (tag & 1) != 0, r.oT.w, cn);
+                    walkStart<false>(wm, wk, ray, (tag & 1) != 0, r.oT.w, cn);
                     walking = true;
                     own = true;
                 }
@@ -211,17 +211,8 @@ __global__ __launch_bounds__(kWfBlock) void k_wf_trace(DevScene s, const WfRay* 
             if (drained) break;
             continue;
         }
-        const bool general = __ballot(walking && wk.p.special) == 0ull;
-        const WalkMem wm = walkMem(s);
-#pragma unroll
-        for (int u = 0; u < kWfRows; ++u) {
-            if (walking && wk.leaf < 0) {
-                if (walkRow<false>(wm, wk, general, cn)) walking = false;
-            }
-        }
-        if (walking && wk.leaf >= 0) {
-            if (walkLeaf<false>(wm, wk, cn)) walking = false;
-        }
+        if (walking && walkRound<false, kWfNodes>(wm, wk, stack, cn)) walking = false;
+        if (!walking && (wk.flags & kWalkPending)) walking = !walkSettle<false>(wm, wk);
         // a walk that ended stores its result in its path
         if (!walking && own) {
             const int path = tag >> 1;
