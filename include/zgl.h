@@ -172,11 +172,11 @@ typedef struct zgl_pass_params {
     int32_t count_bytes;          /* accumulate algorithmic-byte counters (slower) */
     int32_t regen_threshold;      /* naive, light, triple (persistent kernels): lanes of a wave64
                                      still walking the MTBVH when the wave stops to shade and
-                                     reissue rays (1..63).  0 = default: from the triangle count
-                                     n, round(1.4 log2 n - 2) clamped to 4..28 for the naive
-                                     tracer, round(1.3 log2 n - 7) clamped to 1..24 for the
-                                     triple tracer's camera pass, 4 for light paths.  Frames do
-                                     not depend on it. */
+                                     reissue rays (1..63).  0 = default: for the naive tracer and
+                                     the triple tracer's camera pass 1 + (m - 1) f, where m =
+                                     0.7 log2 n - 2.5 clamped to 1..16 for n triangles and f =
+                                     0.2 + u / 48, at most 1, for u samples per resident lane;
+                                     1 for light paths.  Frames do not depend on it. */
 } zgl_pass_params;
 /* ZGL_INTEGRATOR_NAIVE keeps each sample's value (16 bytes) in a context-owned buffer of
  * at most 4 GiB and adds them to the frame in pass order; calls with more passes than fit
@@ -290,15 +290,15 @@ zgl_status zgl_batch_set(zgl_batch* batch, zgl_context* const* contexts, const z
  * (any output may be NULL). */
 zgl_status zgl_batch_plan(const int32_t* film_wh, const zgl_pass_params* params, int32_t n, int64_t* sample_bytes,
                           int32_t* sobol_first, int32_t* sobol_count);
-/* regen_threshold 1..63 for every scene, or 0 (the default): each scene's own zgl_render
- * default for the naive tracer; blocks_per_cu 1..max (0 = max resident);
+/* regen_threshold 1..63 for every scene, or 0 (the default): zgl_render's default for
+ * the naive tracer from each scene's triangles and the whole batch's samples per lane; blocks_per_cu 1..max (0 = max resident);
  * order: a permutation of 0..n-1 giving the launch order (NULL keeps the current one). */
 zgl_status zgl_batch_configure(zgl_batch* batch, int32_t regen_threshold, int32_t blocks_per_cu,
                                const int32_t* order);
 zgl_status zgl_batch_launch(zgl_batch* batch);
 zgl_status zgl_batch_synchronize(zgl_batch* batch);
 /* Autotuner: times the batch (median of `reps` launches after a warm-up) over scene
- * orders (as given / most work first), regeneration thresholds {per scene (0), 8, ..., 32}
+ * orders (as given / most work first), regeneration thresholds {per scene (0), 2, ..., 24}
  * and the two
  * highest blocks-per-CU counts, coordinate by coordinate, and keeps the fastest.  It
  * launches the batch repeatedly: frames of passes that do not start at pass 0

@@ -18,22 +18,30 @@
 
 using namespace zgl;
 
-// zgl_render's default for it (regen_threshold 0).  Frames do not depend on it; the
-// fastest value grows with the length of the walks, which grows with log2 of the
-// triangle count.  Fitted to sweeps on one MI355X over scenes of 36 to 1.3M triangles:
-// the naive tracer was fastest at 4 with 36 triangles, 12 with 852, 16-20 with 10k-100k
-// and 24-28 with 0.8M-1.3M; the triple tracer's camera pass at 1, 8-12 and 16 with 36,
-// 10k and 100k; the light paths at 1-4 at every size.
-enum class WalkKind { Naive, TripleCamera, LightPaths };
-static int defaultThreshold(WalkKind kind, int bvhSize)
+// zgl_render's default for it (regen_threshold 0): how many lanes of a wave may still be
+// walking when the wave stops to shade.  Frames do not depend on it.  Shading early keeps
+// lanes walking and shades with few lanes; it pays with long walks, and with enough units
+// for every lane that a wave which shades can refill its idle lanes: a launch of a few
+// units per lane ends sooner the fewer shading steps its waves make.
+// Sweeps on one MI355X (1024 x 1024, depth 8; ms at the best value, then the time at
+// 4 / 12 / 24 over the best):
+//   16 passes (64 units per lane)          1 pass (4 units per lane)
+//   36 triangles      16.6 at 1: 1.04 1.16 1.43     1.22 at 1:  1.10 1.36 1.73
+//   852               17.8 at 3: 1.00 1.10 1.39     1.70 at 2:  1.04 1.26 1.59
+//   9,828             19.0 at 6: 1.01 1.05 1.32     1.89 at 2:  1.03 1.20 1.51
+//   99,146            22.9 at 12: 1.07 1.00 1.15    2.47 at 4:  1.00 1.11 1.33
+//   1,306,146         31.8 at 12: 1.17 1.00 1.04    4.18 at 12: 1.01 1.00 1.16
+//   819,400 (headline, 1080p, 127 and 8 units per lane)
+//                     27.7 at 12: 1.03 1.00 1.08    2.88 at 4:  1.00 1.12 1.34
+// The rule below is within 4% of the best in all of them and in the triple tracer's
+// camera pass; light paths, short everywhere, were fastest at 1 or 2 at every size.
+static int defaultThreshold(int bvhSize, double unitsPerLane)
 {
     const double l = std::log2((double)std::max(2, (bvhSize + 1) / 2));
-    switch (kind) {
-    case WalkKind::LightPaths: return 4;
-    case WalkKind::TripleCamera: return std::min(24, std::max(1, (int)std::lround(1.3 * l - 7.0)));
-    default: return std::min(28, std::max(4, (int)std::lround(1.4 * l - 2.0)));
-    }
+    const double most = std::min(16.0, std::max(1.0, 0.7 * l - 2.5));
+    return (int)std::lround(1.0 + (most - 1.0) * std::min(1.0, 0.2 + unitsPerLane / 48.0));
 }
+constexpr int kLightPathThreshold = 1;
 // Largest sample-value plus traversal-log buffer of one chunk of the differentiable mode's passes.
 constexpr size_t kAdjointLogBytes = (size_t)8 << 30;
 // Largest total of a batch's per-sample value buffers.
@@ -767,6 +775,15 @@ static PassParams passParams(const zgl_pass_params* p)
     return pp;
 }
 
+// The persistent camera kernels' threshold: the request's, or the default for nPasses passes
+// in a launch of blocksPerCU workgroups of 256 per compute unit.
+static int naiveThreshold(const zgl_context* ctx, int requested, int nPasses, int blocksPerCU)
+{
+    if (requested > 0) return requested;
+    const double lanes = 256.0 * std::max(1, ctx->numCUs * blocksPerCU);
+    return defaultThreshold(ctx->scene.bvhSize, (double)ctx->filmW * ctx->filmH * nPasses / lanes);
+}
+
 // Validates a pass request and builds the per-launch scene view and parameters.
 static void preparePasses(zgl_context* ctx, const zgl_pass_params* p, DevScene& s, PassParams& pp)
 {
@@ -795,8 +812,7 @@ zgl_status zgl_render(zgl_context* ctx, const zgl_pass_params* p)
         float* film = (float*)ctx->film.p;
         if (p->integrator == ZGL_INTEGRATOR_NAIVE) {
             if (!ctx->naiveBlocksPerCU) ctx->naiveBlocksPerCU = naivePersistentBlocksPerCU();
-            const int threshold =
-                p->regen_threshold > 0 ? p->regen_threshold : defaultThreshold(WalkKind::Naive, s.bvhSize);
+            const int threshold = naiveThreshold(ctx, p->regen_threshold, pp.nPasses, ctx->naiveBlocksPerCU);
             // per-sample values of up to 4 GB worth of passes (121 passes at 1080p)
             const size_t perPass = (size_t)ctx->filmW * ctx->filmH * 16;
             const int resPasses = (int)std::max<size_t>(1, std::min<size_t>(pp.nPasses, ((size_t)4 << 30) / perPass));
@@ -827,8 +843,7 @@ zgl_status zgl_render(zgl_context* ctx, const zgl_pass_params* p)
                 hipCheck(launchLight(s, pp, film, cnt, ctx->stream), "light pass");
             } else {
                 if (!ctx->lightBlocksPerCU) ctx->lightBlocksPerCU = lightPersistentBlocksPerCU(false);
-                const int threshold =
-                    p->regen_threshold > 0 ? p->regen_threshold : defaultThreshold(WalkKind::LightPaths, s.bvhSize);
+                const int threshold = p->regen_threshold > 0 ? p->regen_threshold : kLightPathThreshold;
                 hipCheck(launchLightPersistent(s, pp, false, film, (int*)ctx->workCounter.p, threshold,
                                                ctx->numCUs * ctx->lightBlocksPerCU, ctx->stream),
                          "light pass");
@@ -846,8 +861,7 @@ zgl_status zgl_render(zgl_context* ctx, const zgl_pass_params* p)
                 const int resPasses =
                     (int)std::max<size_t>(1, std::min<size_t>(pp.nPasses, ((size_t)4 << 30) / perPass));
                 ctx->ensure(ctx->naiveRes, perPass * resPasses, "sample values");
-                const int threshold =
-                    p->regen_threshold > 0 ? p->regen_threshold : defaultThreshold(WalkKind::TripleCamera, s.bvhSize);
+                const int threshold = naiveThreshold(ctx, p->regen_threshold, pp.nPasses, ctx->tripleBlocksPerCU);
                 hipCheck(launchTriplePersistent(s, pp, film, (float4*)ctx->naiveRes.p, resPasses,
                                                 (int*)ctx->workCounter.p, threshold,
                                                 ctx->numCUs * ctx->tripleBlocksPerCU, ctx->stream),
@@ -859,8 +873,7 @@ zgl_status zgl_render(zgl_context* ctx, const zgl_pass_params* p)
                 hipCheck(launchTripleLPT(sl, pp, film, cnt, ctx->stream), "triple light pass");
             } else {
                 if (!ctx->tripleLightBlocksPerCU) ctx->tripleLightBlocksPerCU = lightPersistentBlocksPerCU(true);
-                const int threshold =
-                    p->regen_threshold > 0 ? p->regen_threshold : defaultThreshold(WalkKind::LightPaths, s.bvhSize);
+                const int threshold = p->regen_threshold > 0 ? p->regen_threshold : kLightPathThreshold;
                 hipCheck(launchLightPersistent(sl, pp, true, film, (int*)ctx->workCounter.p, threshold,
                                                ctx->numCUs * ctx->tripleLightBlocksPerCU, ctx->stream),
                          "triple light pass");
@@ -889,8 +902,7 @@ zgl_status zgl_render_static(zgl_context* ctx, const zgl_pass_params* p)
         const int chunk = (int)std::min<size_t>({(size_t)p->n_passes, kStaticResBytes / perPass,
                                                  (size_t)kStaticChunkPasses});
         if (!ctx->naiveBlocksPerCU) ctx->naiveBlocksPerCU = naivePersistentBlocksPerCU();
-        const int threshold =
-            p->regen_threshold > 0 ? p->regen_threshold : defaultThreshold(WalkKind::Naive, ctx->scene.bvhSize);
+        const int threshold = naiveThreshold(ctx, p->regen_threshold, chunk, ctx->naiveBlocksPerCU);
         int* counter = reinterpret_cast<int*>(base);
         uint32_t* sobol = reinterpret_cast<uint32_t*>(base + kStaticSobolOffset);
         float4* res = reinterpret_cast<float4*>(base + kStaticResOffset);
@@ -1001,7 +1013,7 @@ static void loggedPasses(zgl_context* ctx, const DevScene& s, const PassParams& 
     ctx->logGeneration = 0;
     ctx->ensure(ctx->naiveRes, px * 16 * chunk, "sample values");
     ctx->ensure(ctx->hitLog, px * kHitLogQueries * 8 * chunk, "traversal log");
-    const int threshold = regenThreshold > 0 ? regenThreshold : defaultThreshold(WalkKind::Naive, s.bvhSize);
+    const int threshold = naiveThreshold(ctx, regenThreshold, chunk, ctx->naiveBlocksPerCU);
     for (int k0 = 0; k0 < pp.nPasses; k0 += chunk) {
         PassParams q = pp;
         q.firstPass = pp.firstPass + k0;
@@ -1249,6 +1261,9 @@ static void batchUpload(zgl_batch* b)
     const int n = (int)b->ctxs.size();
     b->host.resize(n);
     b->generations.resize(n);
+    double units = 0.0;
+    for (int i = 0; i < n; i++) units += (double)b->ctxs[i]->filmW * b->ctxs[i]->filmH * b->params[i].n_passes;
+    const double unitsPerLane = units / (256.0 * std::max(1, b->numCUs * b->blocksPerCU));
     for (int i = 0; i < n; i++) b->generations[i] = b->ctxs[i]->generation;
     for (int k = 0; k < n; k++) {
         const int i = b->order[k];
@@ -1256,7 +1271,7 @@ static void batchUpload(zgl_batch* b)
         const zgl_pass_params* p = &b->params[i];
         BatchScene& it = b->host[k];
         it.s = ctx->scene;
-        it.threshold = b->threshold > 0 ? b->threshold : defaultThreshold(WalkKind::Naive, it.s.bvhSize);
+        it.threshold = b->threshold > 0 ? b->threshold : defaultThreshold(it.s.bvhSize, unitsPerLane);
         it.s.sobolTab = (const uint32_t*)b->sobolTab.p;
         it.s.sobolTabFirst = b->sobolFirst;
         it.s.sobolTabCount = b->sobolCount;
@@ -1449,7 +1464,7 @@ zgl_status zgl_batch_tune(zgl_batch* b, int32_t reps, double* best_ms)
             const double t = batchTime(b, reps);
             if (t < best) { best = t; ord = o; }
         }
-        for (int t : {0, 8, 12, 16, 20, 24, 32}) {  // 0: each scene's own default
+        for (int t : {0, 2, 4, 8, 12, 16, 24}) {  // 0: each scene's own default
             config(t, bpc, ord);
             const double tm = batchTime(b, reps);
             if (tm < best) { best = tm; th = t; }
