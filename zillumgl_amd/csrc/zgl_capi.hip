@@ -55,12 +55,12 @@ constexpr int64_t kBatchMaxUnits = (int64_t)INT_MAX - (1 << 24);
 constexpr int kBatchSobolRows = 65537;
 
 // Scratch of zgl_render_static, one array per GPU, held until the process ends:
-// [0, 256) the persistent schedule's unit counters, then the Sobol points of one chunk
+// the persistent schedule's unit counters, then the Sobol points of one chunk
 // of at most kStaticChunkPasses passes (+1 row for dims past 256), then the chunk's
 // per-sample values (16 B per pixel and pass).
-constexpr size_t kStaticScratchBytes = (size_t)128 << 20;
+constexpr size_t kStaticScratchBytes = ((size_t)128 << 20) + kCounterBytes - 256;
 constexpr int kStaticChunkPasses = 256;
-constexpr size_t kStaticSobolOffset = 256;
+constexpr size_t kStaticSobolOffset = kCounterBytes;
 constexpr size_t kStaticResOffset =
     (kStaticSobolOffset + (size_t)(kStaticChunkPasses + 1) * 256 * 4 + 255) & ~(size_t)255;
 constexpr size_t kStaticResBytes = kStaticScratchBytes - kStaticResOffset;
@@ -339,7 +339,7 @@ zgl_status zgl_create(int32_t device, zgl_context** out)
         resolveScratch(device);
         ctx->upload(ctx->sobolM, sobolMatrices(), 256 * 32 * sizeof(uint32_t), "sobol matrices");
         ctx->ensure(ctx->counters, NumCounters * sizeof(unsigned long long), "counters");
-        ctx->ensure(ctx->workCounter, 256, "work counter");
+        ctx->ensure(ctx->workCounter, kCounterBytes, "work counter");
         hipCheck(hipDeviceGetAttribute(&ctx->numCUs, hipDeviceAttributeMultiprocessorCount, device), "attribute");
         hipCheck(hipMemsetAsync(ctx->counters.p, 0, NumCounters * sizeof(unsigned long long), ctx->stream),
                  "counters");
@@ -1326,7 +1326,7 @@ zgl_status zgl_batch_set(zgl_batch* b, zgl_context* const* ctxs, const zgl_pass_
         hipCheck(launchSobolTable((const uint32_t*)ctxs[0]->sobolM.p, (uint32_t*)b->sobolTab.p, b->sobolFirst,
                                   b->sobolCount, b->stream),
                  "sobol table");
-        b->ensure(b->counters, (size_t)n * kUnitRegions * 4, "batch counters");
+        b->ensure(b->counters, (size_t)n * kCounterBytes, "batch counters");
         // every scene's sample values (n_passes x W x H float4), added to its frame in
         // pass order after the persistent kernel
         b->resOffset.resize(n);

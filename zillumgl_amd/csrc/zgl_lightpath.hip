@@ -16,7 +16,9 @@
 //     before the walk in the same order, since a walk draws none;
 //   * a unit is (pass, thread id) of the reference's dispatch: one path for the light
 //     tracer, loopsPerPass paths drawn in turn from one random stream for the triple
-//     light pass; a lane whose unit is done takes the next, one atomic per wave;
+//     light pass; a lane whose unit is done takes the next, one atomic per wave, from the
+//     wave's region first (4.06 -> 3.55 ms on the caustics box with the threshold of 1,
+//     against one counter that all XCDs added to);
 //   * a lane whose connection walk ends splats and starts its extension walk inside the
 //     walk loop.
 // The roulette is written as selects (survival as a flag, the division always
@@ -40,7 +42,10 @@ enum : int {
 
 constexpr int kNodesPerRound = 3;  // as the naive tracer's
 
-__global__ void k_reset_light_counter(int* c) { if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0; }
+__global__ void k_reset_light_counter(int* c)
+{
+    if (threadIdx.x < kUnitRegions && blockIdx.x == 0) c[threadIdx.x * kCounterStride] = 0;
+}
 
 // visible(x, y) (intersection.glsl:429-434) as the walk it issues.
 __device__ __forceinline__ void visibilityRay(vec3 x, vec3 y, Ray& ray, float& dist)
@@ -54,11 +59,11 @@ template <bool TRIPLE>
 __global__ __launch_bounds__(256, 4) void k_lightpath_persistent(DevScene s0, PassParams prm, float* __restrict__ film,
                                                               int* __restrict__ counter, int threshold)
 {
-    const int lane = threadIdx.x & 63;
     Counters cn;
     const int nUnits = prm.pathsPerPass * prm.nPasses;
     const int loops = TRIPLE ? prm.loopsPerPass : 1;
 
+    UnitFetch fetch = unitFetch();
     int phase = kNewUnit;
     int loopsLeft = 0;
     bool walking = false;
@@ -238,18 +243,14 @@ __global__ __launch_bounds__(256, 4) void k_lightpath_persistent(DevScene s0, Pa
         }
         while (!walking && phase == kStart) startPath();
 
-        // new units, one atomic per wave for the lanes that need one
-        const unsigned long long need = __ballot(!walking && phase == kNewUnit);
-        if (need) {
-            const int leader = __ffsll((long long)need) - 1;
-            int base = 0;
-            if (lane == leader) base = atomicAdd(counter, __popcll(need));
-            base = __shfl(base, leader);
-            if (!walking && phase == kNewUnit) {
-                const int idx = base + __popcll(need & ((1ull << lane) - 1ull));
-                if (idx >= nUnits) {
+        // new units for the lanes that need one
+        if (__ballot(!walking && phase == kNewUnit)) {
+            const bool want = !walking && phase == kNewUnit;
+            const int idx = takeUnits(fetch, counter, nUnits, want);
+            if (want) {
+                if (fetch.exhausted >= kUnitRegions) {
                     phase = kDone;
-                } else {
+                } else if (idx >= 0) {
                     const int k = idx / prm.pathsPerPass;
                     const uint32_t pid = (uint32_t)(idx % prm.pathsPerPass);
                     const int spp = prm.firstPass + k;
@@ -294,7 +295,7 @@ hipError_t launchLightPersistent(const DevScene& s, const PassParams& p, bool tr
 {
     if (threshold < 0) threshold = 0;
     if (threshold > 63) threshold = 63;
-    // units are counted in int32 and each wave may take 64 past the end: chunks of passes
+    // units are counted in int32 and each wave may take 64 past each region's end: chunks of passes
     const int chunk = std::max(1, (int)std::min<int64_t>(p.nPasses, ((int64_t)1 << 30) / p.pathsPerPass));
     for (int k0 = 0; k0 < p.nPasses; k0 += chunk) {
         PassParams q = p;

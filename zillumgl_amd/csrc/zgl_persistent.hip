@@ -39,7 +39,6 @@ enum : int {
 // on the headline launch, 24.5 / 23.0 / 22.3 / 21.9 ms on ten batched scenes, 2.78 / 2.69 /
 // 2.70 / 2.80 ms on the material scene.
 constexpr int kNodesPerRound = 3;
-constexpr int kRegions = kUnitRegions;  // unit regions, one per XCD
 
 // Pixel order for the dynamic fetch: 8x8 tiles in row-major tile order.
 __device__ __forceinline__ void pixelOfIndex(int idx, int W, int& x, int& y)
@@ -52,7 +51,10 @@ __device__ __forceinline__ void pixelOfIndex(int idx, int W, int& x, int& y)
 
 }  // namespace
 
-__global__ void k_reset_counter(int* c) { if (threadIdx.x < kRegions && blockIdx.x == 0) c[threadIdx.x] = 0; }
+__global__ void k_reset_counter(int* c)
+{
+    if (threadIdx.x < kUnitRegions && blockIdx.x == 0) c[threadIdx.x * kCounterStride] = 0;
+}
 
 template <bool C> __device__ void flushCountersP(const Counters& cn, unsigned long long* out)
 {
@@ -82,11 +84,9 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
                                           const BatchScene* items, int nScenes, int* sceneCounters, int threshold,
                                           unsigned long long* counters, int2* hitLog)
 {
-    const int lane = threadIdx.x & 63;
     Counters cn;
     int cs = 0;
-    int region = (int)(blockIdx.x % kRegions);  // the workgroup's XCD under round-robin dispatch
-    int exhausted = 0;  // regions of the current scene found used up in a row (the same in every lane)
+    UnitFetch fetch = unitFetch();
 
     int phase = kNewPixel;
     int pix = -1, pass = 0;
@@ -111,7 +111,7 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
         const DevScene& s = BATCH ? items[csu].s : sceneArg(s0);
         const PassParams& prm = BATCH ? items[csu].prm : prm0;
         float4* const res = BATCH ? items[csu].res : res0;
-        int* const pixelCounter = BATCH ? sceneCounters + csu * kRegions : counter0;
+        int* const pixelCounter = BATCH ? sceneCounters + csu * (kUnitRegions * kCounterStride) : counter0;
         const int sceneThreshold = BATCH ? items[csu].threshold : threshold;
         const int W = s.filmW, H = s.filmH;
         const int nIndex = ((W + 7) / 8) * ((H + 7) / 8) * 64;
@@ -312,37 +312,17 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
             }
         }
 
-        // pixels are handed out per wave: one atomic for all lanes that need one.  One
-        // region of 8x8 tiles per XCD (workgroups are dispatched to XCDs round-robin), so
-        // that the waves sharing an L2 start with neighbouring pixels; a wave whose region
-        // is used up moves on to the next, and once all eight are, stops (one scene) or
-        // waits to move to the next scene (batch).
-        const unsigned long long need = __ballot(!walking && phase == kNewPixel);
-        if (need) {
-            const int n = __popcll(need);
-            const int leader = __ffsll((long long)need) - 1;
-            int base = 0;
-            // the wave's region of the image first (one per XCD), then the others
-            const int len = ((nUnits / kRegions + 63) / 64) * 64;
-            const int start = min(nUnits, region * len);
-            const int limit = min(nUnits, start + len);
-            if (lane == leader) base = atomicAdd(pixelCounter + region, n);
-            base = __shfl(base, leader) + start;
-            if (base >= limit) {
-                region = (region + 1) % kRegions;
-                exhausted++;
-            } else {
-                exhausted = 0;
-            }
-            if (!walking && phase == kNewPixel) {
-                const unsigned long long below = need & ((1ull << lane) - 1ull);
-                const int idx = base + __popcll(below);
+        // units are handed out per wave, one region of 8x8 tiles per XCD first, so that the
+        // waves sharing an L2 start with neighbouring pixels; a wave that finds every region
+        // used up stops (one scene) or waits to move to the next scene (batch)
+        if (__ballot(!walking && phase == kNewPixel)) {
+            const bool want = !walking && phase == kNewPixel;
+            const int idx = takeUnits(fetch, pixelCounter, nUnits, want);
+            if (want) {
                 pix = -1;
-                if (exhausted >= kRegions) {
+                if (fetch.exhausted >= kUnitRegions) {
                     phase = BATCH ? kWait : kDone;
-                } else if (idx >= limit) {
-                    // this region is used up: fetch again from the next one
-                } else {
+                } else if (idx >= 0) {
                     const int group = idx >> 6;
                     const int unitPass = group % prm.nPasses;
                     const int pixIdx = (group / prm.nPasses) * 64 + (idx & 63);
@@ -378,8 +358,7 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
             // every lane idle and some waiting: move the wave to the next scene
             if (__ballot(walking || (phase != kWait && phase != kDone)) == 0ull && __ballot(phase == kWait) != 0ull) {
                 cs = csu + 1;
-                region = (int)(blockIdx.x % kRegions);
-                exhausted = 0;
+                fetch = unitFetch();
                 if (phase == kWait) phase = (cs < nScenes) ? kNewPixel : kDone;
                 continue;
             }
@@ -480,10 +459,8 @@ __global__ __launch_bounds__(256, 4) void k_naive_batch(const BatchScene* __rest
 __global__ __launch_bounds__(256, 4) void k_triple_persistent(DevScene s0, PassParams prm, float4* __restrict__ res,
                                                            int* __restrict__ pixelCounter, int threshold)
 {
-    const int lane = threadIdx.x & 63;
     Counters cn;
-    int region = (int)(blockIdx.x % kRegions);
-    int exhausted = 0;
+    UnitFetch fetch = unitFetch();
     const int W = s0.filmW, H = s0.filmH;
     const int nIndex = ((W + 7) / 8) * ((H + 7) / 8) * 64;
     const int nUnits = nIndex * prm.nPasses;
@@ -659,29 +636,14 @@ __global__ __launch_bounds__(256, 4) void k_triple_persistent(DevScene s0, PassP
         }
 
         // samples are handed out per wave, one region of 8x8 tiles per XCD first
-        const unsigned long long need = __ballot(!walking && phase == kNewPixel);
-        if (need) {
-            const int n = __popcll(need);
-            const int leader = __ffsll((long long)need) - 1;
-            int base = 0;
-            const int len = ((nUnits / kRegions + 63) / 64) * 64;
-            const int start = min(nUnits, region * len);
-            const int limit = min(nUnits, start + len);
-            if (lane == leader) base = atomicAdd(pixelCounter + region, n);
-            base = __shfl(base, leader) + start;
-            if (base >= limit) {
-                region = (region + 1) % kRegions;
-                exhausted++;
-            } else {
-                exhausted = 0;
-            }
-            if (!walking && phase == kNewPixel) {
-                const unsigned long long below = need & ((1ull << lane) - 1ull);
-                const int idx = base + __popcll(below);
+        if (__ballot(!walking && phase == kNewPixel)) {
+            const bool want = !walking && phase == kNewPixel;
+            const int idx = takeUnits(fetch, pixelCounter, nUnits, want);
+            if (want) {
                 pix = -1;
-                if (exhausted >= kRegions) {
+                if (fetch.exhausted >= kUnitRegions) {
                     phase = kDone;
-                } else if (idx < limit) {
+                } else if (idx >= 0) {
                     const int group = idx >> 6;
                     const int unitPass = group % prm.nPasses;
                     const int pixIdx = (group / prm.nPasses) * 64 + (idx & 63);
@@ -760,10 +722,6 @@ __global__ void k_reset_counters(int* c, int n)
     if (i < n) c[i] = 0;
 }
 
-}  // namespace zgl
-
-namespace zgl {
-
 hipError_t launchNaivePersistent(const DevScene& s, const PassParams& p, float4* frame, float4* res, int resPasses,
                                  int* pixelCounter, int threshold, int blocks, unsigned long long* counters,
                                  hipStream_t st)
@@ -804,7 +762,7 @@ hipError_t launchNaiveLogged(const DevScene& s, const PassParams& p, float4* res
 hipError_t launchNaiveBatch(const BatchScene* items, int nScenes, int maxPixels, int* sceneCounters, int blocks,
                             hipStream_t st)
 {
-    const int nCounters = nScenes * kRegions;
+    const int nCounters = nScenes * kUnitRegions * kCounterStride;
     hipLaunchKernelGGL(k_reset_counters, dim3((nCounters + 255) / 256), dim3(256), 0, st, sceneCounters, nCounters);
     hipLaunchKernelGGL(k_naive_batch, dim3(blocks), dim3(256), 0, st, items, nScenes, sceneCounters);
     hipLaunchKernelGGL(k_accumulate_batch, dim3((unsigned)((maxPixels + 255) / 256), (unsigned)std::min(nScenes, 4096)),
