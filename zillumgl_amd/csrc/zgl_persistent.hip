@@ -274,8 +274,9 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
                         ls.coef /= pdfSelect;
                         ls.pdf *= pdfSelect;
                         if (ls.pdf > 0.0f) {
-                            vec3 f = materialBSDF(matType, mp, wo, ls.wi, surf.ns, ModeRadiance);
-                            float fp = materialPdf(matType, mp, wo, ls.wi, surf.ns);
+                            vec3 f;
+                            float fp;
+                            materialEval(matType, mp, wo, ls.wi, surf.ns, ModeRadiance, f, fp);
                             float weight = ls.pdf * ls.pdf / (ls.pdf * ls.pdf + fp * fp);
                             pend = f * throughput * satDot(surf.ns, ls.wi) * ls.coef * weight;
                             pendValid = true;

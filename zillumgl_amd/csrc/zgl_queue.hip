@@ -147,8 +147,9 @@ __device__ bool extendPath(const DevScene& s, const PassParams& prm, const Queue
     if (prm.sampleLight) {
         const LightLiSample ls = sampleLightAndEnv<false>(s, pos, ud, us, uniform, portion, cn);
         if (ls.pdf > 0.0f) {
-            const vec3 f = materialBSDF(matType, mp, wo, ls.wi, surf.ns, ModeRadiance);
-            const float fp = materialPdf(matType, mp, wo, ls.wi, surf.ns);
+            vec3 f;
+            float fp;
+            materialEval(matType, mp, wo, ls.wi, surf.ns, ModeRadiance, f, fp);
             const float weight = ls.pdf * ls.pdf / (ls.pdf * ls.pdf + fp * fp);
             accumulate(frame, pix, f * throughput * satDot(surf.ns, ls.wi) * ls.coef * weight);
         }

@@ -423,8 +423,9 @@ __global__ __launch_bounds__(kWfBlock) void k_wf_shade(DevScene s, PassParams pr
                         ls.coef /= pdfSelect;
                         ls.pdf *= pdfSelect;
                         if (ls.pdf > 0.0f) {
-                            vec3 f = materialBSDF(matType, mp, wo, ls.wi, surf.ns, ModeRadiance);
-                            float fp = materialPdf(matType, mp, wo, ls.wi, surf.ns);
+                            vec3 f;
+                            float fp;
+                            materialEval(matType, mp, wo, ls.wi, surf.ns, ModeRadiance, f, fp);
                             float weight = ls.pdf * ls.pdf / (ls.pdf * ls.pdf + fp * fp);
                             pend = f * throughput * satDot(surf.ns, ls.wi) * ls.coef * weight;
                             pendValid = true;
