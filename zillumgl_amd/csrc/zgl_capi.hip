@@ -157,6 +157,7 @@ struct zgl_context {
     // differentiable mode: evaluation point, adjoint input and outputs
     DevBuf evalMat, evalEnv, dFrame, dMat, dEnv;
     DevBuf bvhBounds;  // node bounds of a device-built MTBVH
+    DevBuf envRaw;     // upload staging of the environment map
     DevBuf wide;       // 4-wide tree, then its builder's work memory
     DevBuf gqQueues, gqCounts;  // global-queue path tracer
     int gqBlocksPerCU = 0;
@@ -191,7 +192,7 @@ struct zgl_context {
                          &lightPower, &lightAlias, &lightProb, &env, &envAlias, &envProb, &noise, &sobolM,
                          &sobolTab, &frame, &film, &counters, &scratchRays, &scratchOut, &workCounter,
                          &evalMat, &evalEnv, &dFrame, &dMat, &dEnv, &bvhBounds, &gqQueues, &gqCounts, &wfWork,
-                         &naiveRes, &hitLog, &refSum, &tex, &texScale, &texRaw, &wide};
+                         &naiveRes, &hitLog, &refSum, &tex, &texScale, &texRaw, &envRaw, &wide};
         for (DevBuf* b : all) b->release();
         bvh.release();
     }
@@ -461,20 +462,13 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
                 std::memcpy(o + 6, &r[1], 4);
                 std::memcpy(o + 7, &miss, 4);
             }
-        std::vector<float> tris((size_t)nT * 12, 0.0f);
-        for (int64_t i = 0; i < nT; i++) {
-            float* o = tris.data() + i * 12;
-            for (int v = 0; v < 3; v++)
-                for (int c = 0; c < 3; c++) o[v * 3 + c] = sb->vertices[(size_t)sb->indices[3 * i + v] * 3 + c];
-        }
-        std::vector<uint16_t> env((size_t)w * h * 4, 0);
-        for (size_t i = 0; i < (size_t)w * h; i++)
-            for (int c = 0; c < 3; c++) env[i * 4 + c] = sb->env_rgb16f[i * 3 + c];
-
         if (!deviceBvh) ctx->upload(ctx->rows, rows.data(), rows.size() * 4, "rows");
-        ctx->upload(ctx->tris, tris.data(), tris.size() * 4, "triangles");
         ctx->upload(ctx->indices, sb->indices, (size_t)nT * 12, "indices");
         ctx->upload(ctx->vertices, sb->vertices, (size_t)nV * 12, "vertices");
+        ctx->ensure(ctx->tris, (size_t)nT * 48, "triangles");
+        hipCheck(launchPackTriangles((const float*)ctx->vertices.p, (const int32_t*)ctx->indices.p, nT,
+                                     (float4*)ctx->tris.p, ctx->stream),
+                 "triangles");
         if (deviceBvh) {
             // indices were checked to lie in [0, n_vertices): the int32 buffer reads as uint32
             ctx->ensure(ctx->rows, (size_t)6 * B * 32, "rows");
@@ -508,7 +502,9 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
         ctx->upload(ctx->lightPower, sb->light_power, (size_t)nL * 12, "lightPower");
         ctx->upload(ctx->lightAlias, sb->light_alias, (size_t)nL * 4, "lightAlias");
         ctx->upload(ctx->lightProb, sb->light_prob, (size_t)nL * 4, "lightProb");
-        ctx->upload(ctx->env, env.data(), env.size() * 2, "env");
+        ctx->upload(ctx->envRaw, sb->env_rgb16f, (size_t)w * h * 6, "env");
+        ctx->ensure(ctx->env, (size_t)w * h * 8, "env");
+        hipCheck(launchPackEnv((const uint16_t*)ctx->envRaw.p, (ushort4*)ctx->env.p, (int64_t)w * h, ctx->stream), "env");
         ctx->upload(ctx->envAlias, sb->env_alias, (size_t)(w + 1) * h * 4, "envAlias");
         ctx->upload(ctx->envProb, sb->env_prob, (size_t)(w + 1) * h * 4, "envProb");
         hipCheck(hipStreamSynchronize(ctx->stream), "scene upload");
@@ -718,12 +714,11 @@ zgl_status zgl_trace_any(zgl_context* ctx, const float* rays, const float* tmax,
         checkRays(ctx, n);
         if (n == 0) return;
         if (!rays || !tmax || !occ) invalid("null pointer");
-        std::vector<float> buf((size_t)n * 7);
-        std::memcpy(buf.data(), rays, (size_t)n * 24);
-        std::memcpy(buf.data() + 6 * n, tmax, (size_t)n * 4);
-        ctx->upload(ctx->scratchRays, buf.data(), buf.size() * 4, "rays");
+        ctx->ensure(ctx->scratchRays, (size_t)n * 28, "rays");
         ctx->ensure(ctx->scratchOut, (size_t)n, "trace output");
-        const float* dr = (const float*)ctx->scratchRays.p;
+        float* dr = (float*)ctx->scratchRays.p;
+        hipCheck(hipMemcpyAsync(dr, rays, (size_t)n * 24, hipMemcpyHostToDevice, ctx->stream), "rays");
+        hipCheck(hipMemcpyAsync(dr + 6 * n, tmax, (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream), "rays");
         hipCheck(launchTraceAny(ctx->scene, dr, dr + 6 * n, n, (uint8_t*)ctx->scratchOut.p, ctx->stream),
                  "trace_any");
         hipCheck(hipMemcpyAsync(occ, ctx->scratchOut.p, (size_t)n, hipMemcpyDeviceToHost, ctx->stream), "copy");

@@ -94,6 +94,10 @@ size_t wideWorkBytes(int64_t nTri);
 hipError_t buildWide(const float4* rows, const float4* tris, int64_t nTri, void* work, uint4* slots, hipStream_t st,
                      WideScale& scale);
 hipError_t launchSobolTable(const uint32_t* sobolM, uint32_t* tab, int first, int count, hipStream_t st);
+// A scene's 48-byte triangles from its vertices and indices, and its RGB16F environment
+// texels padded to 8 bytes.
+hipError_t launchPackTriangles(const float* vertices, const int32_t* indices, int64_t n, float4* tris, hipStream_t st);
+hipError_t launchPackEnv(const uint16_t* rgb, ushort4* env, int64_t n, hipStream_t st);
 hipError_t launchFill(float* p, int64_t n, float v, hipStream_t st);
 hipError_t launchSrgbExpand(const uint8_t* rgb, const float* lut, float4* out, int64_t n, hipStream_t st);
 hipError_t launchPostProcess(const float4* frame, float4* out, unsigned char* rgb8, int w, int h, float scale, int tone,
