@@ -327,7 +327,7 @@ const char* zgl_bvh_builder_last_error(const zgl_bvh_builder* builder);
 zgl_status zgl_bvh_builder_upload(zgl_bvh_builder* builder, const float* vertices, int64_t n_vertices,
                                   const uint32_t* indices, int64_t n_triangles);
 /* Build from the uploaded mesh; returns when the build is complete.  subtree_size: nodes
- * with fewer triangles are finished by one wave each (0 = default 256, minimum 3); the
+ * with fewer triangles are finished by one wave each (0 = default 96, minimum 3); the
  * output does not depend on it. */
 zgl_status zgl_bvh_builder_build(zgl_bvh_builder* builder, int32_t subtree_size);
 /* Copy the last build's bounds and hit tables (either may be NULL). */

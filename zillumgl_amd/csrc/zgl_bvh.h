@@ -40,7 +40,9 @@ private:
     size_t workBytes_ = 0;
 };
 
-// Default size below which a subtree is finished by one wave.
-constexpr int kDefaultBvhSubtree = 256;
+// Default size below which a subtree is finished by one wave.  256 / 96: 1.56 / 1.25 ms for
+// 10,040 triangles, 1.81 / 1.50 for 99,146, 2.00 / 1.75 for 205,000, 3.08 / 3.01 for 819,400
+// and 4.12 / 4.09 for 1.3M: shorter serial chains on more waves against one more level.
+constexpr int kDefaultBvhSubtree = 96;
 
 }  // namespace zgl
