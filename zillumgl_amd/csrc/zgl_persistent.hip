@@ -40,13 +40,29 @@ enum : int {
 // 2.70 / 2.80 ms on the material scene.
 constexpr int kNodesPerRound = 3;
 
-// Pixel order for the dynamic fetch: 8x8 tiles in row-major tile order.
-__device__ __forceinline__ void pixelOfIndex(int idx, int W, int& x, int& y)
+// n / d and n % d for 0 <= n < 2^31 and a d that is the same in every lane, whose reciprocal
+// m = (2^32 - 1) / d stays in scalar registers: the product's high half is the quotient or
+// one less.
+__device__ __forceinline__ int divUniform(int n, int d, uint32_t m, int& rem)
 {
-    const int tilesX = (W + 7) / 8;
-    const int tile = idx >> 6, in = idx & 63;
-    x = (tile % tilesX) * 8 + (in & 7);
-    y = (tile / tilesX) * 8 + (in >> 3);
+    int q = (int)__umulhi((uint32_t)n, m);
+    rem = n - q * d;
+    const bool more = rem >= d;
+    q = more ? q + 1 : q;
+    rem = more ? rem - d : rem;
+    return q;
+}
+
+// The pixel and the pass of a work unit: units are in (8x8 tile, pass, pixel of the tile)
+// order, tiles row by row.
+__device__ __forceinline__ void pixelOfUnit(int idx, int tilesX, uint32_t tilesM, int nPasses, uint32_t passesM, int& x,
+                                            int& y, int& pass)
+{
+    const int tile = divUniform(idx >> 6, nPasses, passesM, pass);
+    int col;
+    const int row = divUniform(tile, tilesX, tilesM, col);
+    x = col * 8 + (idx & 7);
+    y = row * 8 + ((idx >> 3) & 7);
 }
 
 }  // namespace
@@ -324,11 +340,10 @@ __device__ __forceinline__ void naiveBody(const DevScene& s0, const PassParams& 
                 if (fetch.exhausted >= kUnitRegions) {
                     phase = BATCH ? kWait : kDone;
                 } else if (idx >= 0) {
-                    const int group = idx >> 6;
-                    const int unitPass = group % prm.nPasses;
-                    const int pixIdx = (group / prm.nPasses) * 64 + (idx & 63);
-                    int x, y;
-                    pixelOfIndex(pixIdx, W, x, y);
+                    int x, y, unitPass;
+                    const int tilesX = (W + 7) / 8;
+                    pixelOfUnit(idx, tilesX, 0xffffffffu / (uint32_t)tilesX, prm.nPasses,
+                                0xffffffffu / (uint32_t)prm.nPasses, x, y, unitPass);
                     if (x < W && y < H) {  // slots of partial edge tiles fetch again next round
                         pix = y * W + x;
                         scr = v2((float)x, (float)y) / v2((float)W, (float)H);
@@ -645,11 +660,10 @@ __global__ __launch_bounds__(256, 4) void k_triple_persistent(DevScene s0, PassP
                 if (fetch.exhausted >= kUnitRegions) {
                     phase = kDone;
                 } else if (idx >= 0) {
-                    const int group = idx >> 6;
-                    const int unitPass = group % prm.nPasses;
-                    const int pixIdx = (group / prm.nPasses) * 64 + (idx & 63);
-                    int x, y;
-                    pixelOfIndex(pixIdx, W, x, y);
+                    int x, y, unitPass;
+                    const int tilesX = (W + 7) / 8;
+                    pixelOfUnit(idx, tilesX, 0xffffffffu / (uint32_t)tilesX, prm.nPasses,
+                                0xffffffffu / (uint32_t)prm.nPasses, x, y, unitPass);
                     if (x < W && y < H) {
                         pix = y * W + x;
                         scr = v2((float)x, (float)y) / v2((float)W, (float)H);
