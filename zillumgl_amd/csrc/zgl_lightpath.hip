@@ -7,7 +7,7 @@
 // vertex (and, for the light tracer, at the light point itself) by a visibility test and
 // a splat into the planar film, and extended by BSDF sampling.  Here each lane runs a
 // path as a state machine whose states end by issuing one walk -- a connection's
-// visibility walk or the extension walk -- and the walks advance a few MTBVH rows per
+// visibility walk or the extension walk -- and the walks advance a few tree nodes per
 // round for the whole wave, as in the naive tracer's persistent kernel:
 //   * a connection's contribution is computed before its visibility walk and splatted
 //     after it if the walk finds no occluder;
