@@ -325,6 +325,21 @@ template <class T> struct TVec4 { T x, y, z, w; };
 // column-major: M * v = c0 v.x + c1 v.y + c2 v.z
 template <class T> struct TMat3 { TVec3<T> c0, c1, c2; };
 
+// n / d and n % d for 0 <= n < 2^31 and a d that is the same in every lane, whose reciprocal
+// m = (2^32 - 1) / d stays in scalar registers: the product's high half is the quotient or
+// one less (n/d - n*m/2^32 = n*(2^32/d - m)/2^32 < 1/2).  Against the compiler's division,
+// about 30 instructions four times per sample: 96.5 -> 96.0 ms on the headline launch, 43.5
+// -> 43.3 ms on an adjoint step.
+ZGL_HD int divUniform(int n, int d, uint32_t m, int& rem)
+{
+    int q = (int)(((uint64_t)(uint32_t)n * m) >> 32);
+    rem = n - q * d;
+    const bool more = rem >= d;
+    q = more ? q + 1 : q;
+    rem = more ? rem - d : rem;
+    return q;
+}
+
 // random.glsl:3-13 -- 32-bit integer hash
 ZGL_HD uint32_t hashU(uint32_t seed)
 {

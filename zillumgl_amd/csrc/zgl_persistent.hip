@@ -41,21 +41,6 @@ enum : int {
 // 2.70 / 2.80 ms on the material scene.
 constexpr int kNodesPerRound = 3;
 
-// n / d and n % d for 0 <= n < 2^31 and a d that is the same in every lane, whose reciprocal
-// m = (2^32 - 1) / d stays in scalar registers: the product's high half is the quotient or
-// one less (n/d - n*m/2^32 = n*(2^32/d - m)/2^32 < 1/2).  Against the compiler's division,
-// about 30 instructions four times per sample: 96.5 -> 96.0 ms on the headline launch, 43.5
-// -> 43.3 ms on an adjoint step.
-__device__ __forceinline__ int divUniform(int n, int d, uint32_t m, int& rem)
-{
-    int q = (int)__umulhi((uint32_t)n, m);
-    rem = n - q * d;
-    const bool more = rem >= d;
-    q = more ? q + 1 : q;
-    rem = more ? rem - d : rem;
-    return q;
-}
-
 // The pixel and the pass of a work unit: units are in (8x8 tile, pass, pixel of the tile)
 // order, tiles row by row.
 __device__ __forceinline__ void pixelOfUnit(int idx, int tilesX, uint32_t tilesM, int nPasses, uint32_t passesM, int& x,
