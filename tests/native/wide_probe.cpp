@@ -49,6 +49,11 @@ extern "C" int64_t probe_wide_build(const float* vertices, const int32_t* indice
     const float* root = g.rows.data();
     g.scale = wideScale(root, root + 3);
     if (!g.scale.ok) return 0;
+    std::vector<int> rowOf((size_t)6 * nTri, -1);
+    for (int k = 0; k < 6 * B; k++) {
+        const int prim = fbitsi(root[(size_t)k * 8 + 6]);
+        if (prim >= 0) rowOf[(size_t)prim * 6 + k / B] = k;
+    }
     std::vector<int> row(1, 0);  // row of every slot
     g.slots.assign(16, 0u);
     for (size_t s = 0; s < row.size(); s++) {
@@ -57,7 +62,7 @@ extern "C" int64_t probe_wide_build(const float* vertices, const int32_t* indice
         if (prim >= 0 && s > 0) {
             std::memcpy(&g.slots[s * 16], &g.tris[(size_t)prim * 12], 36);
             g.slots[s * 16 + 9] = (uint32_t)prim;
-            g.slots[s * 16 + 10] = (uint32_t)row[s];
+            std::memcpy(&g.slots[s * 16 + 10], &rowOf[(size_t)prim * 6], 24);
             continue;
         }
         int out[4] = {row[s], 0, 0, 0};

@@ -46,6 +46,11 @@ def test_batch_sizes(probe, n):
     _compare(probe, ps, n)
 
 
+@pytest.mark.parametrize("name", ["cornell", "duplicates"])
+def test_tables_of_different_trees(probe, name):
+    _compare(probe, wide_rays.loose(scene.pack(wide_rays.padded(SCENES[name]))), 100000)
+
+
 def test_boxes_larger_than_their_triangles(probe):
     ps = scene.pack(scene.config5(32, 32, n=20, env_size=(8, 4)))
     ps.bounds = (ps.bounds + np.array([-1, -1, -1, 1, 1, 1], np.float32) * np.float32(0.05)).astype(np.float32)

@@ -33,6 +33,17 @@ def test_wide_walk_equals_the_rows(probe, name):
     np.testing.assert_array_equal(occ >= 0, ref >= 0)
 
 
+@pytest.mark.parametrize("name", ["cornell", "duplicates", "materials"])
+def test_tables_of_different_trees(probe, name):
+    ps = wide_rays.loose(scene.pack(SCENES[name]))
+    assert probe.build(ps) > 0
+    r = wide_rays.rays(ps, 100000)
+    prim, t, _ = probe.trace(r)
+    ref_prim, ref_t, _ = probe.trace(r, rows_only=True)
+    np.testing.assert_array_equal(prim, ref_prim)
+    np.testing.assert_array_equal(t.view(np.int32), ref_t.view(np.int32))
+
+
 def test_ordinary_rays_hardly_ever_need_the_rows(probe):
     ps = scene.pack(SCENES["spheres"])
     probe.build(ps)

@@ -1,5 +1,6 @@
 """Scenes and rays for the tests of the walk over the 4-wide tree, and the host build of
 that walk (tests/native/wide_probe.cpp)."""
+import copy
 import ctypes as C
 import os
 import subprocess
@@ -75,6 +76,30 @@ def scenes():
     thin[2::3] = thin[0::3] * 0.5 + thin[1::3] * 0.5 + rng.normal(size=(200, 3)) * 1e-5
     soup(thin, "slivers")
     return out
+
+
+def padded(d, n=33):
+    """The scene with a patch of 2 n^2 small triangles in its middle: more triangles than the
+    batch kernels' rule for walking the rows."""
+    out = copy.copy(d)
+    p = np.concatenate([np.asarray(m.positions, np.float64) for m, _ in d.objects])
+    lo, hi = p.min(0), p.max(0)
+    at = lambda x, y, z: tuple(lo + (hi - lo) * np.array([x, y, z]))
+    patch = scene.grid_patch(at(0.4, 0.45, 0.5), at(0.5, 0.45, 0.52), at(0.5, 0.55, 0.54), at(0.4, 0.55, 0.52),
+                             (0, 0, 1), n, 0, n, 0, n)
+    out.objects = list(d.objects) + [(patch, scene.Material())]
+    return out
+
+
+def loose(ps):
+    """The packed scene with tables of different trees: the inner rows of table 0 all get the
+    root's box, the other tables keep theirs."""
+    ps = copy.copy(ps)
+    table = ps.hit_table.copy()
+    first = table.reshape(6, -1, 3)[0]
+    first[first[:, 1] < 0, 0] = first[0, 0]
+    ps.hit_table = table
+    return ps
 
 
 def rays(ps, n, seed=1):

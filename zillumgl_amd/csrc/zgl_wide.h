@@ -56,7 +56,7 @@ namespace zgl {
 //             FP16 offsets from origin, one per child, in units of WalkMem::unit; `child` is
 //             the first child's slot (28 bits) and a leaf bit per child (bits 28..31).
 //             Children lie in consecutive slots; a missing child's box is empty.
-//   triangle: {a.xyz, b.x} {b.yz, c.xy} {c.z, primitive, row of table 0, -} {-}
+//   triangle: {a.xyz, b.x} {b.yz, c.xy} {c.z, primitive, its rows in the six tables}
 // Slot 0 is the root.
 constexpr uint32_t kWideSlotMask = 0x0fffffffu;
 constexpr int kWideLeafBit = (int)0x80000000;
@@ -356,7 +356,7 @@ template <class Stack> ZGL_HD void wideNode(const WalkMem& m, Walk& w, Stack& st
     w.cur = k0 != 0xffffffffu ? wideChild(q0.w, k0) : kWalkNone;
 }
 
-ZGL_HD void wideTri(const WalkMem& m, int slot, vec3& a, vec3& b, vec3& c, int& prim, int& row)
+ZGL_HD void wideTri(const WalkMem& m, int slot, vec3& a, vec3& b, vec3& c, int& prim)
 {
     const WideSlots n = m.wide + (size_t)(uint32_t)(slot & 0x7fffffff) * 4;
     const WideU4 q0 = n[0], q1 = n[1], q2 = n[2];
@@ -364,7 +364,6 @@ ZGL_HD void wideTri(const WalkMem& m, int slot, vec3& a, vec3& b, vec3& c, int& 
     b = v3(bitsf(q0.w), bitsf(q1.x), bitsf(q1.y));
     c = v3(bitsf(q1.z), bitsf(q1.w), bitsf(q2.x));
     prim = (int)q2.y;
-    row = (int)q2.z;
 }
 
 // One step over the wide tree: the node the walk stands at, then the next stacked subtree
@@ -384,9 +383,9 @@ template <class Stack> ZGL_HD void wideStep(const WalkMem& m, Walk& w, Stack& st
 ZGL_HD bool wideLeaf(const WalkMem& m, Walk& w)
 {
     vec3 a, b, c;
-    int prim, row;
+    int prim;
     const int slot = w.leaf;
-    wideTri(m, slot, a, b, c, prim, row);
+    wideTri(m, slot, a, b, c, prim);
     w.leaf = -1;
     float t;
     if (intersectTriangle(a, b, c, w.o, w.d, t)) {
@@ -436,13 +435,19 @@ ZGL_HD bool generalRay(const Walk& w)
            fabsG(w.o.y) <= big && fabsG(w.o.z) <= big;
 }
 
-// Whether the ray passes the reference's box test on every row from the root of table 0
-// down to `row`.
-ZGL_HD bool wideChain(const WalkMem& m, const Walk& w, int row)
+// Whether the ray passes the reference's box test on every row from the root of its table
+// down to the row of the triangle in `slot`.  Tables a caller hands over may be different
+// trees, so another table's ancestors would not do.
+ZGL_HD bool wideChain(const WalkMem& m, const Walk& w, int slot)
 {
     const RayPre p = walkRay(w);
     const bool general = generalRay(w);
-    int k = 0;
+    const int table = cubemapFace(-w.d);
+    const WideSlots n = m.wide + (size_t)(uint32_t)slot * 4;
+    const WideU4 q2 = n[2], q3 = n[3];
+    const int row = (int)(table == 0 ? q2.z : table == 1 ? q2.w : table == 2 ? q3.x : table == 3 ? q3.y
+                          : table == 4 ? q3.z : q3.w);
+    int k = table * m.bvhSize;
     for (;;) {
         float dist;
         int prim, miss;
@@ -461,8 +466,9 @@ template <bool CHAIN> ZGL_HD bool wideSettle(const WalkMem& m, Walk& w)
 {
     if (w.closest < 0) return false;
     vec3 a, b, c;
-    int prim, row;
-    wideTri(m, w.closest, a, b, c, prim, row);
+    int prim;
+    const int slot = w.closest;
+    wideTri(m, slot, a, b, c, prim);
     w.closest = prim;
     const vec3 lo = v3(ieeeMin(ieeeMin(a.x, b.x), c.x), ieeeMin(ieeeMin(a.y, b.y), c.y), ieeeMin(ieeeMin(a.z, b.z), c.z));
     const vec3 hi = v3(ieeeMax(ieeeMax(a.x, b.x), c.x), ieeeMax(ieeeMax(a.y, b.y), c.y), ieeeMax(ieeeMax(a.z, b.z), c.z));
@@ -484,7 +490,7 @@ template <bool CHAIN> ZGL_HD bool wideSettle(const WalkMem& m, Walk& w)
     const bool order = (w.flags & kWalkAny) || w.t2 > w.dist;
     if (!(h >= 0.0f && h >= l && l <= w.t2 && order)) return false;
     // too near an edge of its box for the margins: asked of the ancestors themselves
-    if constexpr (CHAIN) return pairs || wideChain(m, w, row);
+    if constexpr (CHAIN) return pairs || wideChain(m, w, slot);
     return pairs;
 }
 

@@ -1,12 +1,13 @@
 // zgl_wide.hip -- builds a scene's 4-wide tree (zgl_wide.h) on the device from its MTBVH
 // rows and triangles.
 //
-// The walk over the wide tree equals the walk over the rows only if the rows are six
-// threadings of one binary tree over the same leaves: every inner row's box contains its
-// children's, every leaf's box is its triangle's, and every triangle is a leaf of every
-// table.  k_wide_check shows that row by row (rows handed over by a caller may say
-// anything that points forward); a scene that fails it keeps no wide tree and all its
-// rays take the rows.
+// The walk over the wide tree equals the walk over the rows only if each of the six tables
+// threads a binary tree over the same leaves: every inner row's box contains its children's
+// and lies in table 0's root box, every leaf's box is its triangle's, and every triangle is
+// a leaf of every table.  k_wide_check and k_wide_tris show that (rows handed over by a
+// caller may say anything that points forward); a scene that fails it keeps no wide tree
+// and all its rays take the rows.  The six trees need not be the same one: the wide tree
+// is table 0's, and a hit's ancestors are asked in the ray's own table.
 //
 // The tree is built breadth first, a level a launch: a work item is a binary inner row and
 // the slot of its node; its thread gathers the node's up to four children, reserves
@@ -39,14 +40,14 @@ struct WideBuild {
     int n, S, capacity;
     uint4* slots;
     int2* queue[2];     // items of the even and the odd levels: a row and its node's slot
-    uint32_t* mask;     // tables each triangle was met in
+    int* rowOf;         // six per triangle: its row in each table, -1 where it was not met
     WideCounters* c;
 };
 
 // The parts below run over `threads` threads, this one the `tid`-th.
 __device__ __forceinline__ void wideInit(const WideBuild& b, int tid, int threads)
 {
-    for (int g = tid; g < b.n; g += threads) b.mask[g] = 0;
+    for (int64_t g = tid; g < (int64_t)6 * b.n; g += threads) b.rowOf[g] = -1;
     for (int g = tid; g <= kMaxLevels; g += threads) b.c->count[g] = g == 0 ? 1 : 0;
     if (tid < 8) b.c->root[tid] = b.rows[tid];
     if (tid == 0) {
@@ -69,7 +70,7 @@ __device__ __forceinline__ void wideCheck(const WideBuild& b, int tid, int threa
         const int k = (int)g, end = (t + 1) * b.S;  // 6 S fits int32
         const float* r = b.rows + (size_t)k * 8;
         const int prim = __float_as_int(r[6]), miss = __float_as_int(r[7]);
-        bool ok = k != t * b.S || miss == end;
+        bool ok = (k != t * b.S || miss == end) && contains(b.rows, r);
         if (prim >= 0) {
             ok = ok && prim < b.n && miss == k + 1;
             if (ok) {
@@ -78,7 +79,7 @@ __device__ __forceinline__ void wideCheck(const WideBuild& b, int tid, int threa
                     const float lo = fminf(fminf(p[a], p[3 + a]), p[6 + a]), hi = fmaxf(fmaxf(p[a], p[3 + a]), p[6 + a]);
                     ok = ok && r[a] == lo && r[3 + a] == hi;
                 }
-                atomicOr(b.mask + prim, 1u << t);
+                b.rowOf[(size_t)prim * 6 + t] = k;
             }
         } else {
             const int c1 = k + 1;
@@ -98,11 +99,12 @@ __device__ __forceinline__ void wideCheck(const WideBuild& b, int tid, int threa
     if (bad) atomicAdd(&b.c->bad, bad);
 }
 
-__device__ __forceinline__ void wideMask(const WideBuild& b, int tid, int threads)
+// A table has n leaves, so one that holds every triangle holds each of them once.
+__device__ __forceinline__ void wideTris(const WideBuild& b, int tid, int threads)
 {
     int bad = 0;
-    for (int g = tid; g < b.n; g += threads)
-        if (__hip_atomic_load(b.mask + g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0x3fu) bad++;
+    for (int64_t g = tid; g < (int64_t)6 * b.n; g += threads)
+        if (b.rowOf[g] < 0) bad++;
     if (bad) atomicAdd(&b.c->bad, bad);
 }
 
@@ -173,8 +175,10 @@ __device__ __forceinline__ void wideLevel(const WideBuild& b, int level, int ite
                     const float4 p0 = p[0], p1 = p[1], p2 = p[2];
                     d[0] = p0;
                     d[1] = p1;
-                    d[2] = make_float4(p2.x, __int_as_float(prim), __int_as_float(child[j]), 0.0f);
-                    d[3] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    const int* k = b.rowOf + (size_t)prim * 6;
+                    d[2] = make_float4(p2.x, __int_as_float(prim), __int_as_float(k[0]), __int_as_float(k[1]));
+                    d[3] = make_float4(__int_as_float(k[2]), __int_as_float(k[3]), __int_as_float(k[4]),
+                                       __int_as_float(k[5]));
                 }
             }
         }
@@ -189,9 +193,9 @@ __global__ __launch_bounds__(256) void k_wide_check(WideBuild b)
 {
     wideCheck(b, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
-__global__ __launch_bounds__(256) void k_wide_mask(WideBuild b)
+__global__ __launch_bounds__(256) void k_wide_tris(WideBuild b)
 {
-    wideMask(b, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+    wideTris(b, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 __global__ __launch_bounds__(256) void k_wide_level(WideBuild b, int level)
 {
@@ -206,7 +210,7 @@ __global__ __launch_bounds__(256) void k_wide_small(WideBuild b)
     __syncthreads();
     wideCheck(b, threadIdx.x, blockDim.x);
     __syncthreads();
-    wideMask(b, threadIdx.x, blockDim.x);
+    wideTris(b, threadIdx.x, blockDim.x);
     __syncthreads();
     if (__hip_atomic_load(&b.c->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
     for (int level = 0; level < kMaxLevels; level++) {
@@ -226,7 +230,7 @@ size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // above triangles alone and a third of that above those: n + 2 n / 3 slots.
 int64_t wideCapacity(int64_t n) { return n + (2 * n) / 3 + 16; }
 
-size_t wideWorkBytes(int64_t n) { return align256(sizeof(WideCounters)) + 2 * align256((size_t)n * 8 + 8) + (size_t)n * 4; }
+size_t wideWorkBytes(int64_t n) { return align256(sizeof(WideCounters)) + 2 * align256((size_t)n * 8 + 8) + (size_t)n * 24; }
 
 hipError_t buildWide(const float4* rows, const float4* tris, int64_t nTri, void* work, uint4* slots, hipStream_t st,
                      WideScale& scale)
@@ -249,7 +253,7 @@ hipError_t buildWide(const float4* rows, const float4* tris, int64_t nTri, void*
         b.queue[i] = reinterpret_cast<int2*>(p);
         p += align256((size_t)n * 8 + 8);
     }
-    b.mask = reinterpret_cast<uint32_t*>(p);
+    b.rowOf = reinterpret_cast<int*>(p);
     const bool small = n <= kSmallBuild;
     if (small) {
         hipLaunchKernelGGL(k_wide_small, dim3(1), dim3(256), 0, st, b);
@@ -258,7 +262,7 @@ hipError_t buildWide(const float4* rows, const float4* tris, int64_t nTri, void*
         hipLaunchKernelGGL(k_wide_init, dim3(perTri), dim3(256), 0, st, b);
         hipLaunchKernelGGL(k_wide_check, dim3((unsigned)std::min<int64_t>(8192, ((int64_t)6 * S + 255) / 256)), dim3(256),
                            0, st, b);
-        hipLaunchKernelGGL(k_wide_mask, dim3(perTri), dim3(256), 0, st, b);
+        hipLaunchKernelGGL(k_wide_tris, dim3(perTri), dim3(256), 0, st, b);
     }
     WideCounters host;
     for (int level = 0; level < kMaxLevels;) {
