@@ -3,6 +3,7 @@
 // an MTBVH as the device builder does (the slots in breadth-first order) and returns the
 // slot count, or 0 where the scene has no wide tree; probe_wide_trace walks rays and
 // repeats over the rows those the wide walk cannot vouch for, as the kernels do.
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <vector>
@@ -21,9 +22,29 @@ struct Tree {
     std::vector<float> rows, tris;
     std::vector<uint32_t> slots;
     WideScale scale;
+    WideMargins margins;
     int bvhSize;
 };
 Tree g;
+
+// k_wide_tris' sums, one triangle after the other
+void collect(WideStats& st, const WideTriClass& c)
+{
+    if (c.kind == kWideTriSmall) {
+        st.x = std::max(st.x, fbits(c.x));
+        st.diagonal = std::max(st.diagonal, fbits(c.diagonal));
+    }
+    if (c.kind != kWideTriLarge) return;
+    st.edge = std::max(st.edge, fbits(c.edge));
+    int i = 0;
+    while (i < kWidePlaneSlots && st.key[i] != 0 && st.key[i] != c.key) i++;
+    if (c.key == 0 || i == kWidePlaneSlots) {
+        st.overflow = 1;
+        return;
+    }
+    st.sine[i] = st.key[i] == 0 ? fbits(c.sine) : std::min(st.sine[i], fbits(c.sine));
+    st.key[i] = c.key;
+}
 }  // namespace
 
 extern "C" int64_t probe_wide_build(const float* vertices, const int32_t* indices, int64_t nTri, const float* bounds,
@@ -54,6 +75,9 @@ extern "C" int64_t probe_wide_build(const float* vertices, const int32_t* indice
         const int prim = fbitsi(root[(size_t)k * 8 + 6]);
         if (prim >= 0) rowOf[(size_t)prim * 6 + k / B] = k;
     }
+    WideStats st{};
+    for (int64_t i = 0; i < nTri; i++) collect(st, wideClassify(&g.tris[i * 12], g.scale.bound));
+    g.margins = wideMargins(st, g.scale);
     std::vector<int> row(1, 0);  // row of every slot
     g.slots.assign(16, 0u);
     for (size_t s = 0; s < row.size(); s++) {
@@ -76,7 +100,8 @@ extern "C" int64_t probe_wide_build(const float* vertices, const int32_t* indice
 }
 
 // rowsOnly: every ray over the rows.  stats: [0] walks over the wide tree, [1] of them repeated over the rows, [2] nodes,
-// [3] triangles, [4] largest stack, [5] rays that took the rows from the start
+// [3] triangles, [4] largest stack, [5] rays that took the rows from the start, [6] walks that
+// ran out of stack, [7] rows, [8] walks made again that drop nothing
 extern "C" void probe_wide_trace(const float* rays, int64_t n, const float* tmax, int any, int rowsOnly,
                                  int32_t* prim, float* t, int64_t* stats)
 {
@@ -87,31 +112,44 @@ extern "C" void probe_wide_trace(const float* rays, int64_t n, const float* tmax
     m.bvhSize = g.bvhSize;
     m.unit = g.scale.unit;
     m.bound = g.scale.bound;
-    m.slack = 4.0f * g.scale.pad;
+    m.rel = g.margins.rel;
+    m.slack = g.margins.slack;
+    m.margins = &g.margins;
     for (int64_t i = 0; i < n; i++) {
         f32::Walk w;
         f32::walkStart(m, w, v3(rays[i], rays[n + i], rays[2 * n + i]), v3(rays[3 * n + i], rays[4 * n + i], rays[5 * n + i]),
                        any != 0, any ? tmax[i] : 1e8f);
         HostStack st;
         stats[w.closest == f32::kWalkRedo ? 5 : 0]++;
-        if (w.closest == f32::kWalkRedo) {
-            f32::walkRows(m, w);
-        } else {
+        if (w.closest == f32::kWalkRedo) f32::walkRows(m, w);
+        while (!(w.flags & f32::kWalkRows)) {
             bool done = false;
             while (!done) {
                 if (w.cur >= 0 && w.cur != f32::kWalkNone) stats[2]++;
                 f32::wideStep(m, w, st);
                 if (w.sp > stats[4]) stats[4] = w.sp;
+                if (w.closest == f32::kWalkRedo) stats[6]++;
                 if (w.leaf >= 0) { stats[3]++; done = f32::wideLeaf(m, w); }
                 done = done || (w.cur == f32::kWalkNone && w.sp == 0);
             }
-            if (w.closest != -1 && !f32::wideSettle<true>(m, w)) f32::walkRows(m, w);
-            if (w.flags & f32::kWalkRows) stats[1]++;
+            const int how = w.closest == -1 ? f32::kSettled : f32::wideSettle<true>(m, w);
+            if (how == f32::kSettled) break;
+            stats[how == f32::kSettleWhole ? 8 : 1]++;
+            if (how == f32::kSettleWhole) f32::wideWhole(w);
+            else f32::walkRows(m, w);
         }
         uint32_t rows = 0, tests = 0;
         if (w.flags & f32::kWalkRows)
             while (!f32::rowsStep(m, w, f32::generalRay(w), rows, tests)) {}
+        stats[7] += rows;
         prim[i] = w.closest;
         t[i] = w.dist;
     }
+}
+
+// The margins of the built tree.
+extern "C" void probe_wide_margins(float out[5])
+{
+    const float v[5] = {g.margins.rel, g.margins.slack, g.margins.grow, g.margins.growRel, g.margins.reach};
+    std::memcpy(out, v, sizeof(v));
 }

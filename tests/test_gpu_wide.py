@@ -17,8 +17,8 @@ def probe(tmp_path_factory):
     return wide_rays.Probe(tmp_path_factory.mktemp("wide"))
 
 
-def _compare(probe, ps, n):
-    r = wide_rays.rays(ps, n)
+def _compare(probe, ps, n, r=None):
+    r = wide_rays.rays(ps, n) if r is None else r
     ctx = render.Context(0)
     try:
         ctx.upload(ps)
@@ -27,7 +27,7 @@ def _compare(probe, ps, n):
         np.testing.assert_array_equal(prim, ref[0])
         np.testing.assert_array_equal(t.view(np.int32), ref[1].view(np.int32))
         np.testing.assert_array_equal(b, ref[2])
-        tm = wide_rays.limits(ps, n)
+        tm = wide_rays.limits(ps, r.shape[1])
         probe.build(ps)
         want, _, _ = probe.trace(r, tm, rows_only=True)
         np.testing.assert_array_equal(ctx.trace_any(r, tm), want >= 0)
@@ -44,6 +44,13 @@ def test_batches_equal_the_rows(probe, name):
 def test_batch_sizes(probe, n):
     ps = scene.pack(scene.config5(32, 32, n=20, env_size=(8, 4)))  # above the rule's 2,048 triangles
     _compare(probe, ps, n)
+
+
+@pytest.mark.parametrize("name,scale,turned", wide_rays.LARGE)
+def test_rays_nearly_in_a_triangles_plane(probe, name, scale, turned):
+    ps = scene.pack(wide_rays.scaled(wide_rays.padded(SCENES[name]), scale, turned))
+    r = wide_rays.grazing(ps, 100000)
+    _compare(probe, ps, 0, np.concatenate([r, wide_rays.flattened(r)], 1))
 
 
 @pytest.mark.parametrize("name", ["cornell", "duplicates"])

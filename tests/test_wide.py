@@ -33,6 +33,80 @@ def test_wide_walk_equals_the_rows(probe, name):
     np.testing.assert_array_equal(occ >= 0, ref >= 0)
 
 
+@pytest.mark.parametrize("name,scale,turned", wide_rays.LARGE)
+def test_rays_nearly_in_a_triangles_plane(probe, name, scale, turned):
+    ps = scene.pack(wide_rays.scaled(SCENES[name], scale, turned))
+    assert probe.build(ps) > 0
+    r = wide_rays.grazing(ps, 100000)
+    for rays in (r, wide_rays.flattened(r)):
+        prim, t, _ = probe.trace(rays)
+        ref_prim, ref_t, _ = probe.trace(rays, rows_only=True)
+        np.testing.assert_array_equal(prim, ref_prim)
+        np.testing.assert_array_equal(t.view(np.int32), ref_t.view(np.int32))
+        tm = wide_rays.limits(ps, rays.shape[1])
+        occ, _, _ = probe.trace(rays, tm)
+        ref, _, _ = probe.trace(rays, tm, rows_only=True)
+        np.testing.assert_array_equal(occ >= 0, ref >= 0)
+
+
+def _hits(tri, o, d):
+    """intersectTriangle (src/shader/intersection.glsl:63-109) in FP32, operation by operation:
+    the mask of hits, t and |det|."""
+    dot = lambda x, y: (x[:, 0] * y[:, 0] + x[:, 1] * y[:, 1]) + x[:, 2] * y[:, 2]
+
+    def cross(x, y):
+        return np.stack([x[:, 1] * y[:, 2] - x[:, 2] * y[:, 1], x[:, 2] * y[:, 0] - x[:, 0] * y[:, 2],
+                         x[:, 0] * y[:, 1] - x[:, 1] * y[:, 0]], 1)
+    a, ab, ac = tri[:, 0], tri[:, 1] - tri[:, 0], tri[:, 2] - tri[:, 0]
+    p, ao = cross(d, ac), o - a
+    det = dot(ab, p)
+    ao = np.where((det < 0)[:, None], -ao, ao)
+    det = np.abs(det)
+    q = cross(ao, ab)
+    u, v = dot(ao, p), dot(d, q)
+    with np.errstate(all="ignore"):
+        t = dot(ac, q) / det
+        hit = (det >= np.float32(1e-6)) & (u >= 0) & (u <= det) & (v >= 0) & (u + v <= det) & (t > 0)
+    return hit, t, det
+
+
+@pytest.mark.parametrize("size", [0.03, 0.3, 3.0, 300.0])
+@pytest.mark.parametrize("flat", [False, True])
+def test_how_far_a_hit_lies_from_its_triangle(size, flat):
+    """The bound that the walk's margins are made from (zgl_wide.h): the point at t lies within
+    14.7 u X R / |det| + 4 u (R + t + edges) of the triangle's plane, and for a triangle in a
+    plane of constant z the distance is right to (4 / s + 8) u."""
+    g = np.random.default_rng(11)
+    n, u = 400000, 2.0 ** -24
+    tri = (g.uniform(-1, 1, (n, 1, 3)) * 5 * size + g.normal(size=(n, 3, 3)) * size).astype(np.float32)
+    if flat:
+        tri[:, 1:, 2] = tri[:, :1, 2]
+    t64 = tri.astype(np.float64)
+    ab, ac = t64[:, 1] - t64[:, 0], t64[:, 2] - t64[:, 0]
+    normal = np.cross(ab, ac)
+    area = np.linalg.norm(normal, axis=1)
+    normal /= area[:, None]
+    a = g.uniform(0, 2 * np.pi, n)[:, None]
+    along = ab / np.linalg.norm(ab, axis=1)[:, None]
+    off = np.clip(10 ** g.uniform(-0.5, 4, n) * 1e-6 / area, 0, 0.5) * g.choice([-1, 1], n)
+    d = along * np.cos(a) + np.cross(normal, along) * np.sin(a) + normal * off[:, None]
+    d = (d / np.linalg.norm(d, axis=1)[:, None]).astype(np.float32)
+    on = (t64 * g.dirichlet([1, 1, 1], n)[..., None]).sum(1)
+    o = (on - d.astype(np.float64) * g.uniform(0, 10 * size, (n, 1))).astype(np.float32)
+    hit, t, det = _hits(tri, o, d)
+    assert hit.sum() > 1000
+    t64, ab, ac, normal, area = t64[hit], ab[hit], ac[hit], normal[hit], area[hit]
+    o, d, t, det = o[hit].astype(np.float64), d[hit].astype(np.float64), t[hit].astype(np.float64), det[hit].astype(np.float64)
+    x = np.linalg.norm(ab, axis=1) * np.linalg.norm(ac, axis=1)
+    r = np.linalg.norm(o - t64[:, 0], axis=1)
+    edges = np.linalg.norm(ab, axis=1) + np.linalg.norm(ac, axis=1)
+    beside = np.abs(((o + t[:, None] * d - t64[:, 0]) * normal).sum(1))
+    assert (beside <= 14.7 * u * x * r / det + 4 * u * (r + t + edges)).all()
+    if flat:
+        exact = ((t64[:, 0] - o) * normal).sum(1) / (d * normal).sum(1)
+        assert (np.abs(t - exact) <= (4 * x / area + 8) * u * np.abs(exact)).all()
+
+
 @pytest.mark.parametrize("name", ["cornell", "duplicates", "materials"])
 def test_tables_of_different_trees(probe, name):
     ps = wide_rays.loose(scene.pack(SCENES[name]))

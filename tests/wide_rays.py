@@ -34,7 +34,7 @@ class Probe:
         r = np.ascontiguousarray(rays, np.float32)
         n = r.shape[1]
         tm = np.zeros(n, np.float32) if tmax is None else np.ascontiguousarray(tmax, np.float32)
-        prim, t, st = np.empty(n, np.int32), np.empty(n, np.float32), np.zeros(6, np.int64)
+        prim, t, st = np.empty(n, np.int32), np.empty(n, np.float32), np.zeros(9, np.int64)
         self.lib.probe_wide_trace(p(r, C.c_float), C.c_int64(n), p(tm, C.c_float), int(tmax is not None),
                                   int(rows_only), p(prim, C.c_int32), p(t, C.c_float), p(st, C.c_int64))
         return prim, t, st
@@ -100,6 +100,55 @@ def loose(ps):
     first[first[:, 1] < 0, 0] = first[0, 0]
     ps.hit_table = table
     return ps
+
+
+def scaled(d, k, turned=False):
+    """The scene k times as large, turned about two axes if asked (no face stays in a plane of
+    constant x, y or z)."""
+    c, s, e, f = np.cos(0.6), np.sin(0.6), np.cos(0.9), np.sin(0.9)
+    turn = np.array([[c, -s, 0], [s, c, 0], [0, 0, 1]]) @ np.array([[1, 0, 0], [0, e, -f], [0, f, e]]) if turned else np.eye(3)
+
+    def moved(mesh):
+        m = copy.copy(mesh)
+        m.positions = np.ascontiguousarray(((np.asarray(mesh.positions, np.float64) @ turn.T) * k).astype(np.float32))
+        return m
+    out = copy.copy(d)
+    out.objects = [(moved(m), x) for m, x in d.objects]
+    out.lights = [(moved(m), x) for m, x in d.lights]
+    return out
+
+
+def grazing(ps, n, seed=7):
+    """Rays nearly in the plane of a triangle, 1e-7 to 0.1 off it, from on it, in front of it
+    or behind: the FP32 distance of such a hit is far off, and can lie in front of the
+    triangle's own box."""
+    g = np.random.default_rng(seed)
+    t = ps.vertices[ps.indices[g.integers(0, len(ps.indices), n)]].astype(np.float64)
+    o = (t * g.dirichlet([1, 1, 1], n)[..., None]).sum(1)
+    ab, ac = t[:, 1] - t[:, 0], t[:, 2] - t[:, 0]
+    unit = lambda v: v / np.maximum(np.linalg.norm(v, axis=1), 1e-30)[:, None]
+    normal, along = unit(np.cross(ab, ac)), unit(ab)
+    a = g.uniform(0, 2 * np.pi, n)[:, None]
+    d = along * np.cos(a) + np.cross(normal, along) * np.sin(a)
+    d = unit(d + normal * (10 ** g.uniform(-7, -1, n) * g.choice([-1, 1], n))[:, None])
+    size = np.linalg.norm(ps.vertices.max(0).astype(np.float64) - ps.vertices.min(0))
+    o += d * (g.choice([0, 1e-4], n) - g.choice([0, 0, 0.1, 0.3], n) * size)[:, None]
+    return np.ascontiguousarray(np.concatenate([o.T, d.T]).astype(np.float32))
+
+
+def flattened(r, seed=3):
+    """The rays with one component of their directions below 1e-6."""
+    g = np.random.default_rng(seed)
+    r, n = r.copy(), r.shape[1]
+    r[3 + g.integers(0, 3, n), np.arange(n)] = g.choice([0, 1e-7, -9e-7, 1e-20], n)
+    r[3:] /= np.maximum(np.linalg.norm(r[3:].astype(np.float64), axis=0), 1e-9).astype(np.float32)
+    return r
+
+
+# scene, scale, turned: sizes at which walks that drop subtrees at a fixed distance beyond
+# the hit, or test a flattened ray's box on all three axes, return other hits than the rows
+LARGE = [("cornell", 10, False), ("cornell", 100, True), ("materials", 555, True), ("caustics", 1000, True),
+         ("tessellated", 100, False), ("tessellated", 555, True), ("spheres", 100, False), ("duplicates", 10, True)]
 
 
 def rays(ps, n, seed=1):

@@ -481,6 +481,7 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
         }
         // a device too full for the wide tree renders over the rows, with the same results
         WideScale wideScale{};
+        WideMargins wideMargins{};
         const size_t wideBytes = (size_t)wideCapacity(nT) * 64;
         bool wideFits = true;
         try {
@@ -492,7 +493,8 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
         }
         if (wideFits)
             hipCheck(buildWide((const float4*)ctx->rows.p, (const float4*)ctx->tris.p, nT,
-                               (char*)ctx->wide.p + wideBytes, (uint4*)ctx->wide.p, ctx->stream, wideScale),
+                               (char*)ctx->wide.p + wideBytes, (uint4*)ctx->wide.p, ctx->stream, wideScale,
+                               wideMargins),
                      "wide tree build");
         ctx->upload(ctx->normals, sb->normals, (size_t)nV * 12, "normals");
         ctx->upload(ctx->texcoords, sb->texcoords, (size_t)sb->n_texcoords * 8, "texcoords");
@@ -514,8 +516,8 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
         s.tris = (const float4*)ctx->tris.p;
         s.wide = wideScale.ok ? (const uint4*)ctx->wide.p : nullptr;
         s.wideUnit = wideScale.unit;
-        s.wideSlack = 4.0f * wideScale.pad;
         s.wideBound = wideScale.bound;
+        s.wideMargins = wideMargins;
         s.indices = (const int32_t*)ctx->indices.p;
         s.vertices = (const float*)ctx->vertices.p;
         s.normals = (const float*)ctx->normals.p;

@@ -41,7 +41,8 @@ struct DevScene {
     const float4* rows;          // 6 * bvhSize * 2
     const float4* tris;          // nTriangles * 3
     const uint4* wide;           // 4-wide tree of the same leaves (zgl_wide.h), or null
-    float wideUnit, wideSlack, wideBound;
+    float wideUnit, wideBound;
+    WideMargins wideMargins;
     const int32_t* indices;      // 3 per triangle
     const float* vertices;       // 3 per vertex
     const float* normals;        // 3 per vertex
@@ -115,7 +116,7 @@ template <bool C> ZGL_D void cnt(Counters& c, uint32_t b) { if (C) c.bytes += b;
 template <bool C> ZGL_D WalkMem walkMem(const DevScene& s)
 {
     WalkMem m{(GRows)s.rows, (GRows)s.tris, C ? (WideSlots) nullptr : (WideSlots)s.wide, s.bvhSize, s.wideUnit,
-              s.wideSlack, s.wideBound};
+              s.wideBound, s.wideMargins.rel, s.wideMargins.slack, &s.wideMargins};
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("" : "+s"(m.rows), "+s"(m.tris), "+s"(m.wide));
 #endif
@@ -218,15 +219,17 @@ template <bool C, int kNodes> ZGL_D bool walkRound(const WalkMem& m, Walk& w, Ld
     }
     return done;
 }
-// Settles a walk that ended kWalkPending; false when it goes on, over the rows.  The
-// resumable schedules walk those rays among the others, with the wave's next rounds; a
-// walk by one lane (CHAIN) would hold up its wave for a hundred rows and asks the hit's
-// ancestors first.
+// Settles a walk that ended kWalkPending; false when it goes on, over the wide tree or the
+// rows.  The resumable schedules walk those rays among the others, with the wave's next
+// rounds; a walk by one lane (CHAIN) would hold up its wave for a hundred rows and asks
+// the hit's ancestors first.
 template <bool CHAIN> ZGL_D bool walkSettle(const WalkMem& m, Walk& w)
 {
     w.flags &= ~kWalkPending;
-    if (wideSettle<CHAIN>(m, w)) return true;
-    walkRows(m, w);
+    const int how = wideSettle<CHAIN>(m, w);
+    if (how == kSettled) return true;
+    if (how == kSettleWhole) wideWhole(w);
+    else walkRows(m, w);
     return false;
 }
 // A whole walk by one lane: the closest hit's primitive (dist 1e8 on a miss), or any.
@@ -237,6 +240,7 @@ ZGL_D int walkAll(const DevScene& s, vec3 o, vec3 d, bool any, float& dist)
     LdsStack st = walkStack();
     Walk w;
     walkStart(m, w, o, d, any, dist);
+    if (!any && w.closest != kWalkRedo && !wideDrops(m, w)) wideWhole(w);
     do {
         while (!walkRound<false, 1>(m, w, st, cn)) {}
     } while ((w.flags & kWalkPending) && !walkSettle<true>(m, w));

@@ -88,11 +88,12 @@ struct BatchScene {
 
 // The 4-wide tree of a scene's rows and triangles (zgl_wide.hip): slots holds
 // wideCapacity(n) slots of 64 bytes, work wideWorkBytes(n) bytes.  scale.ok is false where
-// the scene has no wide tree (its rays then take the rows).  Synchronises the stream.
+// the scene has no wide tree (its rays then take the rows); margins: up to what distance its
+// walks keep subtrees.  Synchronises the stream.
 int64_t wideCapacity(int64_t nTri);
 size_t wideWorkBytes(int64_t nTri);
 hipError_t buildWide(const float4* rows, const float4* tris, int64_t nTri, void* work, uint4* slots, hipStream_t st,
-                     WideScale& scale);
+                     WideScale& scale, WideMargins& margins);
 hipError_t launchSobolTable(const uint32_t* sobolM, uint32_t* tab, int first, int count, hipStream_t st);
 // A scene's 48-byte triangles from its vertices and indices, and its RGB16F environment
 // texels padded to 8 bytes.

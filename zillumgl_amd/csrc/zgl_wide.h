@@ -22,29 +22,62 @@
 // the leaf's.  So a leaf whose margins exceed 8 u (Ty + Tz) passes together with all its
 // ancestors.
 //   * The walk here visits every leaf whose box passes in the reference (its boxes
-//     contain the exact ones, with room for the rounding of both sides), so it tests
-//     every triangle the reference may test, and more.
+//     contain the exact ones, with room for the rounding of both sides), up to the
+//     distance at which it drops subtrees (wideLimit).
 //   * Let W be its closest hit at t, t2 the next larger hit distance it met (the ray's
-//     limit if none), b the entry distance of W's exact box.  If W's box passes with those
-//     margins, t < t2 and b <= t2, then whenever the reference's walk comes to W its
-//     distance is still at least t2: W is tested, and nothing is nearer.  So the
-//     reference's closest hit is W whatever order it visits the leaves in.  Where only the
-//     margins fail (about one hit in a thousand), the reference's box test can be made on
-//     W's ancestors themselves (CHAIN), a fifth of a walk over the rows.
-//   * Without a hit the reference has none either.  For an any-hit ray one hit that passes
-//     with these margins and b <= the limit shows that it is occluded.
-// Measured: 47 rows become 13 nodes and 3 triangles a ray on the headline scene; the
-// 64-pass 1080p launch went from 169 to 114 ms, one 720p pass of a 205,000-triangle scene
-// from 15.7 to 2.0 ms (see the last paragraph), ten batched scenes from 28.8 to 22.2 ms.
-// A node step is about 110 vector instructions for four boxes (fma_mix reads the FP16
-// planes in place) against 45 for one row.
+//     limit if none), b the entry distance of W's exact box, and T a little more than t.  No
+//     triangle in a dropped subtree has a hit distance of T or less (below).  If W's box
+//     passes with those margins, t < t2, b <= t2 and b <= T, then whenever the
+//     reference's walk comes to W its distance is still above t and at least b: W is
+//     tested, and nothing is nearer.  So the reference's closest hit is W whatever order
+//     it visits the leaves in.  Where only the margins fail (about one hit in a thousand),
+//     the reference's box test can be made on W's ancestors themselves (CHAIN), a fifth of
+//     a walk over the rows.
+//   * Without a hit the reference has none either.  For an any-hit ray, which drops
+//     nothing, one hit that passes with these margins and b <= the limit shows that it is
+//     occluded.
+//
+// How far a hit lies from its triangle.  Write X = |ab| |ac|, R = |a - o|, |d| = 1, and det as
+// intersectTriangle computes it.  Cramer's identity det ao + num d = u ab + v ac holds
+// exactly for exact determinants; the computed ones, all of them small beside their terms
+// where the ray is nearly edge-on, are each off by at most 3.66 u times the product of
+// their three vectors' lengths.  With u, v >= 0 and u + v <= det the point o + t d is
+// therefore within 14.7 u X R / det (and a few u R) of the triangle.  Edge-on, where det
+// comes near its cut-off of 1e-6, that is 0.9 X R: not small unless X is, and t can lie
+// well in front of the triangle's own box.  So no fixed widening of the distance lets a
+// walk drop subtrees; each triangle has to be of one of four kinds (wideClassify):
+//   * small: X at most kWideSmall and its box's diagonal at most bound / 8.  The ray is in
+//     the box at its entry e and within 0.9 X R of the triangle at t, so e - t is at most
+//     the diagonal and 1.03 * 0.9 X (t + diagonal) / (1 - 0.9 X).
+//   * flat: in a plane of constant x, y or z.  Every product of det, num and of the errors
+//     then carries the same component of d or of o - a, t is accurate to 6 u / s whatever
+//     the angle (s the sine of the angle at a) and e is at most the flat slab's distance.
+//   * never hit: det stays below its cut-off for every ray.
+//   * large: everything else.  det >= g s X (but for 0.4%) where g = |d.N|.  Of the four terms
+//     of the offset between the point at t and the triangle two are along d and two along
+//     ab and ac, each pair 7.4 u (R + edge / 2) / (g s) at most; only the latter move the
+//     ray's entry, by their component on the entry's axis over d's, which is at least the
+//     smallest component h of d.  So e - t <= (7.4 (1 / h + 2) / (g s) + 10 / h) u (t + 1.5
+//     edge), and a ray with g s (h - 10 K u) >= 7.6 K u (1 + 2 h) for every large triangle's
+//     plane (wideClear) has e - t <= (t + 1.5 edge) / K.  A walk of another ray, one in a
+//     few hundred, is made again and drops no subtree (wideWhole).  The planes are few
+//     where a scene has large triangles, walls and floors; of a scene with more than
+//     kWidePlanes no walk drops any.  Dropping nothing costs 25 to 50% on the caustics box,
+//     whose rays go on through the sphere's back.
+// wideMargins makes from the scene's largest X, diagonal and edge the limit (rel, slack)
+// up to which a walk has to keep subtrees.
+//
+// Measured: 47 rows become 13 nodes and 3 triangles a ray on the headline scene.  A node
+// step is about 110 vector instructions for four boxes (fma_mix reads the FP16 planes in
+// place) against 45 for one row.
 //
 // Rays the argument does not cover take the reference's rows from the start: nearly
-// axis-parallel ones (RayPre::mode != 0), two components below 1e-6, not finite, from far
-// outside the scene, or with a direction shorter than 0.5.  A ray with one component
-// below 1e-6, whose box test drops that axis' slab, is covered with the remaining pair's
-// margin; the reference's walk of such a ray visits every box of a slice through the scene
-// (15 ms for one ray on a 205,000-triangle scene), the walk here a ray's worth.
+// axis-parallel ones (RayPre::mode != 0), components below 1e-6, not finite, from far
+// outside the scene, or with a direction longer than 1 or shorter (any-hits: than 0.5).
+// For a ray with one component below 1e-6 the reference's test drops that axis' slab, and
+// its walk visits every box of a slice through the scene (15 ms for one ray on a
+// 205,000-triangle scene).  Boxes further from the ray on that axis than a hit can lie
+// beside its triangle are left out of that walk (rowHit).
 #pragma once
 
 #include "zgl_box.h"
@@ -82,6 +115,21 @@ typedef const GFloat4* GRows;
 // A stacked subtree: its parent's child word and its key (entry distance and child number).
 struct WalkEntry { uint32_t word, key; };
 
+// A plane of large triangles (wideClear).  kWideClear is K at the top of the file: a larger
+// one drops more and walks more rays twice.
+constexpr double kWideClear = 64.0;
+constexpr int kWidePlanes = 16;
+struct WidePlane { float x, y, z, w; };
+
+// Up to what distance a walk keeps subtrees, for which rays, and how far beside its triangle
+// a hit can lie (see the top of the file).
+struct WideMargins {
+    float rel, slack;            // the limit is rel * distance + slack (infinite: nothing is dropped)
+    float grow, growRel, reach;  // wideGrowth
+    int nPlanes;
+    WidePlane planes[kWidePlanes];
+};
+
 // The scene as a walk sees it.
 struct WalkMem {
     GRows rows;        // the reference's row tables
@@ -89,8 +137,9 @@ struct WalkMem {
     WideSlots wide;    // null: every ray takes the rows
     int bvhSize;
     float unit;        // world length of one FP16 unit of the planes (a power of two)
-    float slack;       // added to the distance when a box is compared with it
     float bound;       // largest absolute coordinate of the scene's box
+    float rel, slack;  // margins->rel, ->slack
+    const WideMargins* margins;
 };
 
 // Sizes derived from the scene's box: bound = its largest absolute coordinate, pad = what
@@ -121,6 +170,140 @@ ZGL_HD WideScale wideScale(const float* lo, const float* hi)
     w.unit = bitsf((e - 14u) << 23);
     w.ok = true;
     return w;
+}
+
+// What a scene's triangles are to the bound at the top of the file: the largest X and box
+// diagonal of the small ones, the longest edge of the large ones, and the large ones' planes,
+// each with the smallest sine at a.  The floats are nonnegative and kept as their bits, whose
+// order is theirs.
+constexpr float kWideSmall = 0.25f;
+constexpr int kWidePlaneSlots = 64;
+struct WideStats {
+    uint32_t x, diagonal, edge;
+    uint32_t overflow;  // planes that found no slot
+    uint32_t key[kWidePlaneSlots], sine[kWidePlaneSlots];  // key 0: free
+};
+enum : int { kWideTriSmall, kWideTriFlat, kWideTriNever, kWideTriLarge, kWideTriBad };
+struct WideTriClass {
+    int kind;
+    float x, diagonal, edge, sine;  // rounded up, the sine down
+    uint32_t key;                   // a large one's plane (wideNormal)
+};
+// p: the corners a, b, c.
+ZGL_HD WideTriClass wideClassify(const float* p, float bound)
+{
+    WideTriClass r{kWideTriBad, 0.0f, 0.0f, 0.0f, 0.0f, 0u};
+    // the edges as intersectTriangle rounds them
+    double ab[3], ac[3], ab2 = 0.0, ac2 = 0.0, bc2 = 0.0, diag2 = 0.0;
+    bool flat = false;
+    for (int c = 0; c < 3; c++) {
+        ab[c] = p[3 + c] - p[c];
+        ac[c] = p[6 + c] - p[c];
+        ab2 += ab[c] * ab[c];
+        ac2 += ac[c] * ac[c];
+        bc2 += (ac[c] - ab[c]) * (ac[c] - ab[c]);
+        const double less = ab[c] < ac[c] ? ab[c] : ac[c], more = ab[c] < ac[c] ? ac[c] : ab[c];
+        const double extent = (more > 0.0 ? more : 0.0) - (less < 0.0 ? less : 0.0);
+        diag2 += extent * extent;
+        flat = flat || (ab[c] == 0.0 && ac[c] == 0.0);
+    }
+    const double n[3] = {ab[1] * ac[2] - ab[2] * ac[1], ab[2] * ac[0] - ab[0] * ac[2], ab[0] * ac[1] - ab[1] * ac[0]};
+    const double x = __builtin_sqrt(ab2 * ac2), len = __builtin_sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+    if (!(x <= 1e30)) return r;  // not finite
+    r.x = (float)x * 1.00001f;
+    r.diagonal = (float)__builtin_sqrt(diag2) * 1.00001f;
+    // |det| <= 1.7321 |n| + 3.66 u 1.7321 X for directions of components up to 1
+    if (1.74 * len + 4e-7 * x < 0.9e-6) r.kind = kWideTriNever;
+    else if (flat && len >= 0.0625 * x) r.kind = kWideTriFlat;
+    else r.kind = r.x <= kWideSmall && r.diagonal <= bound * 0.125f ? kWideTriSmall : kWideTriLarge;
+    if (r.kind != kWideTriLarge) return r;
+    const double longest = ab2 > ac2 ? (ab2 > bc2 ? ab2 : bc2) : (ac2 > bc2 ? ac2 : bc2);
+    r.edge = (float)__builtin_sqrt(longest) * 1.00001f;
+    r.sine = (float)(len / x) * 0.99999f;
+    if (!(len > 0.0)) return r;  // no plane: key 0
+    // the normal's largest component, and the other two over it in steps of 2^-11
+    const double m[3] = {n[0] < 0.0 ? -n[0] : n[0], n[1] < 0.0 ? -n[1] : n[1], n[2] < 0.0 ? -n[2] : n[2]};
+    const int k = m[0] >= m[1] && m[0] >= m[2] ? 0 : m[1] >= m[2] ? 1 : 2;
+    const double ni = k == 0 ? n[1] : n[0], nj = k == 2 ? n[1] : n[2], nk = k == 0 ? n[0] : k == 1 ? n[1] : n[2];
+    r.key = ((uint32_t)(k + 1) << 26) | ((uint32_t)(int)(ni / nk * 2048.0 + 2048.5) << 13) |
+            (uint32_t)(int)(nj / nk * 2048.0 + 2048.5);
+    return r;
+}
+
+// The unit normal a key stands for, within 2^-11 / sqrt 2 of every normal of that key up to
+// its sign.
+ZGL_HD void wideNormal(uint32_t key, double n[3])
+{
+    const int k = (int)(key >> 26) - 1, i = k == 0 ? 1 : 0, j = k == 2 ? 1 : 2;
+    n[k] = 1.0;
+    n[i] = ((double)((key >> 13) & 0x1fffu) - 2048.0) / 2048.0;
+    n[j] = ((double)(key & 0x1fffu) - 2048.0) / 2048.0;
+    const double s = 1.0 / __builtin_sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+    for (int c = 0; c < 3; c++) n[c] *= s;
+}
+
+inline WideMargins wideMargins(const WideStats& st, const WideScale& sc)
+{
+    WideMargins m{};
+    const double x = bitsf(st.x), c = 0.9 * x, diagonal = bitsf(st.diagonal), edge = bitsf(st.edge);
+    // planes: keys next to each other (one plane's triangles round apart) make one
+    const double cell = 3.46e-4;
+    double n[kWidePlanes][3], away[kWidePlanes], sine[kWidePlanes];
+    bool drop = st.overflow == 0;
+    for (int i = 0; i < kWidePlaneSlots && drop; i++) {
+        if (st.key[i] == 0) continue;
+        double v[3], d = 0.0;
+        wideNormal(st.key[i], v);
+        int at = 0;
+        for (; at < m.nPlanes; at++) {
+            const double dot = v[0] * n[at][0] + v[1] * n[at][1] + v[2] * n[at][2], sign = dot < 0.0 ? -1.0 : 1.0;
+            double d2 = 0.0;
+            for (int a = 0; a < 3; a++) d2 += (v[a] - sign * n[at][a]) * (v[a] - sign * n[at][a]);
+            d = __builtin_sqrt(d2) + cell;
+            if (d <= 5.0 * cell) break;
+        }
+        if (at == kWidePlanes) {
+            drop = false;
+        } else if (at == m.nPlanes) {
+            for (int a = 0; a < 3; a++) n[at][a] = v[a];
+            away[at] = cell;
+            sine[at] = bitsf(st.sine[i]);
+            m.nPlanes++;
+        } else {
+            away[at] = d > away[at] ? d : away[at];
+            sine[at] = sine[at] < bitsf(st.sine[i]) ? sine[at] : bitsf(st.sine[i]);
+        }
+    }
+    if (!drop) {
+        m.nPlanes = 0;
+        m.rel = 1.0f;
+        m.slack = __builtin_inff();
+        m.growRel = 1e9f;  // past the scene's end
+        return m;
+    }
+    double rel = 1.03 * c / (1.0 - c), abs = 1.03 * diagonal / (1.0 - c);
+    const bool large = edge > 0.0;
+    if (large) {
+        rel = rel > 1.05 / kWideClear ? rel : 1.05 / kWideClear;
+        abs = abs > 1.6 * edge / kWideClear ? abs : 1.6 * edge / kWideClear;
+    }
+    m.rel = (float)(1.0009765625 * (1.0 + rel) * 1.00001);
+    m.slack = (float)((16.0 * sc.pad + abs) * 1.00001);
+    // beside the triangle on an axis with |d_axis| < 1e-6, where of the four terms of the
+    // identity's error two are left: small ones 0.22 X (2 R + diagonal) / (1 - 0.22 X); large
+    // ones that the ray is clear of with h = 1/16, (R + edge) / 500; flat ones 22 u R / s; the
+    // ray's own drift and the box's rounding
+    m.grow = (float)(sc.bound * 2.44140625e-4);
+    m.growRel = (float)((large && 0.5 * x < 2.1e-3 ? 2.1e-3 : 0.5 * x) * 1.00001);
+    m.reach = (float)((diagonal > edge ? diagonal : edge) * 1.00001);
+    for (int i = 0; i < m.nPlanes; i++) {
+        const double k = sine[i] / (7.6 * kWideClear * 5.9604644775390625e-08);
+        m.planes[i].x = (float)(n[i][0] * k);
+        m.planes[i].y = (float)(n[i][1] * k);
+        m.planes[i].z = (float)(n[i][2] * k);
+        m.planes[i].w = (float)((away[i] * 1.02 + 1e-6) * k);
+    }
+    return m;
 }
 
 ZGL_HD float halfToFloat(uint32_t h)
@@ -220,6 +403,9 @@ enum : int {
     kWalkAny = 1,      // any-hit: ends at the first hit
     kWalkRows = 2,     // over the reference's rows
     kWalkPending = 4,  // ended over the wide tree with a result still to be settled
+    kWalkNear = 8,     // over the rows: leaves out boxes beyond wideGrowth on a dropped axis
+    kWalkWhole = 16,   // drops no subtree: dist stays at its limit, t2 is the closest hit's
+    kWalkDoubt = 32,   // kWalkWhole: another hit lies within W's T
 };
 constexpr int kWalkNone = 0x7fffffff;  // Walk::cur: at no slot, the next stacked one is due
 constexpr int kWalkRedo = -2;          // Walk::closest: to be walked over the rows
@@ -241,11 +427,51 @@ ZGL_HD void walkIdle(Walk& w)
     w.cur = 0; w.leaf = -1; w.sp = 0; w.closest = -1; w.flags = 0;
 }
 
+// Whether the ray is far enough from edge-on to every large triangle, h being the smallest
+// component of its direction that enters a box test.
+ZGL_HD bool wideClear(const WalkMem& m, const Walk& w, float h)
+{
+    const WideMargins& mg = *m.margins;
+    bool clear = true;
+    const float k = h - 10.0f * (float)kWideClear * 5.9604644775390625e-08f, one = 1.0f + 2.0f * h;
+    for (int i = 0; i < mg.nPlanes; i++) {
+        const WidePlane p = mg.planes[i];
+        clear = clear && (fabsG((w.d.x * p.x + w.d.y * p.y) + w.d.z * p.z) - p.w) * k >= one;
+    }
+    return clear;
+}
+
+// The reach and the length of direction that the bounds hold for; false for NaN.
+ZGL_HD bool wideCovers(const WalkMem& m, const Walk& w, float shortest)
+{
+    const float one = 1.0f - 1e-6f, reach = 4.0f * m.bound, dd = dot(w.d, w.d);
+    return m.wide && fabsG(w.d.x) <= one && fabsG(w.d.y) <= one && fabsG(w.d.z) <= one && dd >= shortest &&
+           dd <= 1.02f && fabsG(w.o.x) <= reach && fabsG(w.o.y) <= reach && fabsG(w.o.z) <= reach;
+}
+
+// Whether a closest-hit walk of the ray may drop subtrees.
+ZGL_HD bool wideDrops(const WalkMem& m, const Walk& w)
+{
+    return wideClear(m, w, ieeeMin(ieeeMin(fabsG(w.d.x), fabsG(w.d.y)), fabsG(w.d.z)));
+}
+// Starts (again) over the wide tree, dropping nothing.
+ZGL_HD void wideWhole(Walk& w)
+{
+    w.flags = kWalkWhole;
+    w.dist = w.t2 = 1e8f;
+    w.cur = 0;
+    w.leaf = -1;
+    w.sp = 0;
+    w.closest = -1;
+}
+
 // Starts (again) over the reference's rows.
 ZGL_HD void walkRows(const WalkMem& m, Walk& w)
 {
-    w.inv = v3(1.0f / w.d.x, 1.0f / w.d.y, 1.0f / w.d.z);
+    const float eps = 1e-6f;
+    const int dropped = (fabsG(w.d.x) < eps ? 1 : 0) + (fabsG(w.d.y) < eps ? 1 : 0) + (fabsG(w.d.z) < eps ? 1 : 0);
     w.flags = (w.flags & kWalkAny) | kWalkRows;
+    if (dropped == 1 && wideCovers(m, w, 0.98f) && wideClear(m, w, 0.0625f)) w.flags |= kWalkNear;
     if (!(w.flags & kWalkAny)) w.dist = 1e8f;
     w.cur = cubemapFace(-w.d) * m.bvhSize;
     w.sp = w.cur + m.bvhSize;
@@ -256,37 +482,30 @@ ZGL_HD void walkRows(const WalkMem& m, Walk& w)
 // has to take the rows ends at its first step, to be redone.
 ZGL_HD void walkStart(const WalkMem& m, Walk& w, vec3 o, vec3 d, bool any, float tmax)
 {
-    const float eps = 1e-6f, one = 1.0f - eps;
+    const float eps = 1e-6f;
     w.o = o;
     w.d = d;
     w.dist = tmax;
     w.t2 = tmax;
     w.flags = any ? kWalkAny : 0;
-    const float ax = fabsG(d.x), ay = fabsG(d.y), az = fabsG(d.z);
-    const bool tx = ax < eps, ty = ay < eps, tz = az < eps;
-    const float reach = 4.0f * m.bound;
-    // NaN fails the comparisons on o and on d.d
-    const bool wide = m.wide && ax <= one && ay <= one && az <= one && (ax * ax + ay * ay) + az * az >= 0.25f &&
-                      !((tx && ty) || (ty && tz) || (tx && tz)) && fabsG(o.x) <= reach && fabsG(o.y) <= reach &&
-                      fabsG(o.z) <= reach;
-    // a dropped axis (below 1e-6) keeps a finite reciprocal: its slab is tested here, and
-    // over the scene a component below 1e-15 moves the ray by less than the pad
-    const float tiny = 1e-15f;
-    w.inv = v3(1.0f / (ax < tiny ? __builtin_copysignf(tiny, d.x) : d.x),
-               1.0f / (ay < tiny ? __builtin_copysignf(tiny, d.y) : d.y),
-               1.0f / (az < tiny ? __builtin_copysignf(tiny, d.z) : d.z));
+    // an any-hit drops nothing, so its direction may be shorter
+    const bool wide = wideCovers(m, w, any ? 0.25f : 0.98f) && fabsG(d.x) >= eps && fabsG(d.y) >= eps && fabsG(d.z) >= eps;
+    w.inv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
     w.cur = wide ? 0 : kWalkNone;
     w.leaf = -1;
     w.sp = 0;
     w.closest = wide ? -1 : kWalkRedo;
 }
 
+// The distance boxes are compared with: a subtree that begins beyond it holds no hit as
+// near as W's T.
+ZGL_HD float wideLimit(const WalkMem& m, const Walk& w)
+{
+    return __builtin_fmaf(w.dist, m.rel, m.slack);
+}
+
 ZGL_HD uint32_t umin32(uint32_t a, uint32_t b) { return a < b ? a : b; }
 ZGL_HD uint32_t umax32(uint32_t a, uint32_t b) { return a < b ? b : a; }
-
-// The distance boxes are compared with: dist widened by 2^-10 and the slack, so that a
-// triangle slightly nearer than its box's computed entry is still tested.
-ZGL_HD float wideLimit(const WalkMem& m, const Walk& w) { return __builtin_fmaf(w.dist, 1.0009765625f, m.slack); }
 
 // The slot of the child a key names, with the leaf bit at a triangle.
 ZGL_HD int wideChild(uint32_t word, uint32_t key)
@@ -379,6 +598,12 @@ template <class Stack> ZGL_HD void wideStep(const WalkMem& m, Walk& w, Stack& st
     if (w.cur == kWalkNone && w.sp > 0) widePop(m, w, st);
 }
 
+// W's T for a hit at t.
+ZGL_HD float wideNear(const WalkMem& m, float t)
+{
+    return __builtin_fmaf(t, 1.0009765625f, m.bound * 1.52587890625e-05f);
+}
+
 // Tests the triangle put by; true when it ends the walk (an any-hit).
 ZGL_HD bool wideLeaf(const WalkMem& m, Walk& w)
 {
@@ -389,11 +614,19 @@ ZGL_HD bool wideLeaf(const WalkMem& m, Walk& w)
     w.leaf = -1;
     float t;
     if (intersectTriangle(a, b, c, w.o, w.d, t)) {
-        const bool nearer = t < w.dist;
+        const bool whole = (w.flags & kWalkWhole) != 0;
+        const float best = whole ? w.t2 : w.dist;
+        const bool nearer = t < best;
         w.closest = nearer ? slot : w.closest;
         if (w.flags & kWalkAny) return nearer;
-        w.t2 = nearer ? w.dist : ieeeMin(w.t2, t);
-        w.dist = nearer ? t : w.dist;
+        if (whole) {
+            w.t2 = nearer ? t : best;
+            const bool doubt = (nearer ? best : t) <= wideNear(m, w.t2);
+            w.flags = doubt ? w.flags | kWalkDoubt : nearer ? w.flags & ~kWalkDoubt : w.flags;
+        } else {
+            w.t2 = nearer ? w.dist : ieeeMin(w.t2, t);
+            w.dist = nearer ? t : w.dist;
+        }
     }
     return false;
 }
@@ -413,8 +646,10 @@ ZGL_HD RayPre walkRay(const Walk& w)
     return p;
 }
 
-// The reference's box test on the row k.
-ZGL_HD bool rowHit(const WalkMem& m, const RayPre& p, bool general, int k, float& boxDist, int& prim, int& miss)
+// The reference's box test on the row k; `general`: boxHitGeneral does.  A box further than
+// `grow` from the origin on an axis that the test drops holds no hit and counts as missed.
+ZGL_HD bool rowHit(const WalkMem& m, const RayPre& p, bool general, float grow, int k, float& boxDist, int& prim,
+                   int& miss)
 {
     const GRows row = m.rows + (size_t)(uint32_t)k * 2;
     const GFloat4 lo = row[0], hi = row[1];
@@ -422,8 +657,22 @@ ZGL_HD bool rowHit(const WalkMem& m, const RayPre& p, bool general, int k, float
     prim = fbitsi(hi.z);
     miss = fbitsi(hi.w);
     bool hit = boxHitGeneral(bMin, bMax, p, boxDist);
-    if (!general) hit = boxHit(bMin, bMax, p, boxDist);
+    if (!general) {
+        hit = boxHit(bMin, bMax, p, boxDist);
+        hit = hit && !(p.nx && (bMin.x - grow > p.o.x || bMax.x + grow < p.o.x));
+        hit = hit && !(p.ny && (bMin.y - grow > p.o.y || bMax.y + grow < p.o.y));
+        hit = hit && !(p.nz && (bMin.z - grow > p.o.z || bMax.z + grow < p.o.z));
+    }
     return hit;
+}
+
+// How far beside its triangle a hit nearer than the distance can lie on the axis that a
+// kWalkNear ray's box test drops.
+ZGL_HD float wideGrowth(const WalkMem& m, const Walk& w)
+{
+    const WideMargins& mg = *m.margins;
+    const float r = ((fabsG(w.o.x) + fabsG(w.o.y)) + fabsG(w.o.z)) + 1.74f * m.bound;
+    return mg.grow + mg.growRel * (ieeeMin(r, 1.4f * (w.dist + mg.reach)) + mg.reach);
 }
 
 // Rays for which the three-slab box test alone is the reference's (RayPre::special false).
@@ -441,7 +690,6 @@ ZGL_HD bool generalRay(const Walk& w)
 ZGL_HD bool wideChain(const WalkMem& m, const Walk& w, int slot)
 {
     const RayPre p = walkRay(w);
-    const bool general = generalRay(w);
     const int table = cubemapFace(-w.d);
     const WideSlots n = m.wide + (size_t)(uint32_t)slot * 4;
     const WideU4 q2 = n[2], q3 = n[3];
@@ -451,7 +699,7 @@ ZGL_HD bool wideChain(const WalkMem& m, const Walk& w, int slot)
     for (;;) {
         float dist;
         int prim, miss;
-        if (!rowHit(m, p, general, k, dist, prim, miss)) return false;
+        if (!rowHit(m, p, true, 0.0f, k, dist, prim, miss)) return false;
         if (k == row) return true;
         const GFloat4 first = m.rows[(size_t)(uint32_t)(k + 1) * 2 + 1];
         k = row < fbitsi(first.w) ? k + 1 : fbitsi(first.w);
@@ -459,12 +707,18 @@ ZGL_HD bool wideChain(const WalkMem& m, const Walk& w, int slot)
 }
 
 // Whether the reference's walk finds the triangle this one found (see the top of the
-// file); false where the walk has to be repeated over the rows.  `closest` becomes the
-// primitive either way, before the ancestors are asked: set after that loop, ROCm 7.2's
-// compiler left the slot in it for the lanes that had been through the loop.
-template <bool CHAIN> ZGL_HD bool wideSettle(const WalkMem& m, Walk& w)
+// file), or how the walk has to be repeated.  `closest` becomes the primitive before the
+// ancestors are asked: set after that loop, ROCm 7.2's compiler left the slot in it for the lanes that had
+// been through the loop.
+enum : int { kSettled, kSettleWhole, kSettleRows };
+template <bool CHAIN> ZGL_HD int wideSettle(const WalkMem& m, Walk& w)
 {
-    if (w.closest < 0) return false;
+    if (w.closest < 0) return kSettleRows;
+    if (!(w.flags & (kWalkAny | kWalkWhole)) && !wideDrops(m, w)) return kSettleWhole;
+    if (w.flags & kWalkWhole) {
+        w.dist = w.t2;
+        w.t2 = w.flags & kWalkDoubt ? w.dist : 1e8f;
+    }
     vec3 a, b, c;
     int prim;
     const int slot = w.closest;
@@ -476,22 +730,17 @@ template <bool CHAIN> ZGL_HD bool wideSettle(const WalkMem& m, Walk& w)
     const vec3 mn = v3(ieeeMin(ta.x, tb.x), ieeeMin(ta.y, tb.y), ieeeMin(ta.z, tb.z));
     const vec3 mx = v3(ieeeMax(ta.x, tb.x), ieeeMax(ta.y, tb.y), ieeeMax(ta.z, tb.z));
     // 8 u T per axis
-    const float u8 = 4.76837158203125e-07f, eps = 1e-6f;
+    const float u8 = 4.76837158203125e-07f;
     const float nx = (m.bound + fabsG(w.o.x)) * fabsG(w.inv.x) * u8;
     const float ny = (m.bound + fabsG(w.o.y)) * fabsG(w.inv.y) * u8;
     const float nz = (m.bound + fabsG(w.o.z)) * fabsG(w.inv.z) * u8;
-    const bool cx = mx.y - mn.z > ny + nz, cy = mx.z - mn.x > nz + nx, cz = mx.x - mn.y > nx + ny;
-    const bool tx = fabsG(w.d.x) < eps, ty = fabsG(w.d.y) < eps, tz = fabsG(w.d.z) < eps;
-    // an axis below 1e-6 drops out of the slabs and leaves one pair
-    const float ninf = -__builtin_inff(), pinf = __builtin_inff();
-    const float l = ieeeMax(ieeeMax(tx ? ninf : mn.x, ty ? ninf : mn.y), tz ? ninf : mn.z);
-    const float h = ieeeMin(ieeeMin(tx ? pinf : mx.x, ty ? pinf : mx.y), tz ? pinf : mx.z);
-    const bool pairs = tx ? cx : ty ? cy : tz ? cz : (cx && cy && cz);
-    const bool order = (w.flags & kWalkAny) || w.t2 > w.dist;
-    if (!(h >= 0.0f && h >= l && l <= w.t2 && order)) return false;
+    const bool pairs = mx.y - mn.z > ny + nz && mx.z - mn.x > nz + nx && mx.x - mn.y > nx + ny;
+    const float l = ieeeMax(ieeeMax(mn.x, mn.y), mn.z), h = ieeeMin(ieeeMin(mx.x, mx.y), mx.z);
+    const bool order = (w.flags & kWalkAny) || (w.t2 > w.dist && l <= wideNear(m, w.dist));
+    if (!(h >= 0.0f && h >= l && l <= w.t2 && order)) return kSettleRows;
     // too near an edge of its box for the margins: asked of the ancestors themselves
-    if constexpr (CHAIN) return pairs || wideChain(m, w, slot);
-    return pairs;
+    if constexpr (CHAIN) return pairs || wideChain(m, w, slot) ? kSettled : kSettleRows;
+    return pairs ? kSettled : kSettleRows;
 }
 
 // Up to four of the reference's rows and the triangle of a leaf met on the way, with the
@@ -501,6 +750,7 @@ template <bool CHAIN> ZGL_HD bool wideSettle(const WalkMem& m, Walk& w)
 ZGL_HD bool rowsStep(const WalkMem& m, Walk& w, bool general, uint32_t& rows, uint32_t& tests)
 {
     const RayPre p = walkRay(w);
+    const float grow = w.flags & kWalkNear ? wideGrowth(m, w) : __builtin_inff();
     int leaf = -1;
 #pragma nounroll
     for (int u = 0; u < 4; u++) {
@@ -508,7 +758,7 @@ ZGL_HD bool rowsStep(const WalkMem& m, Walk& w, bool general, uint32_t& rows, ui
             rows++;
             float boxDist;
             int prim, miss;
-            const bool hit = rowHit(m, p, general, w.cur, boxDist, prim, miss);
+            const bool hit = rowHit(m, p, general, grow, w.cur, boxDist, prim, miss);
             const bool take = hit && !(boxDist > w.dist);
             leaf = take && prim >= 0 ? prim : leaf;
             w.cur = take ? (prim >= 0 ? w.cur : w.cur + 1) : miss;

@@ -33,6 +33,7 @@ struct WideCounters {
     int bad;                     // rows that fail the check
     int slots;                   // slots reserved
     int count[kMaxLevels + 1];   // items of each level
+    WideStats stats;
 };
 struct WideBuild {
     const float* rows;  // 6 tables of S rows
@@ -49,10 +50,15 @@ __device__ __forceinline__ void wideInit(const WideBuild& b, int tid, int thread
 {
     for (int64_t g = tid; g < (int64_t)6 * b.n; g += threads) b.rowOf[g] = -1;
     for (int g = tid; g <= kMaxLevels; g += threads) b.c->count[g] = g == 0 ? 1 : 0;
+    for (int g = tid; g < kWidePlaneSlots; g += threads) {
+        b.c->stats.key[g] = 0;
+        b.c->stats.sine[g] = 0x7f7fffffu;
+    }
     if (tid < 8) b.c->root[tid] = b.rows[tid];
     if (tid == 0) {
         b.c->bad = 0;
         b.c->slots = 1;
+        b.c->stats.x = b.c->stats.diagonal = b.c->stats.edge = b.c->stats.overflow = 0;
         b.queue[0][0] = make_int2(0, 0);  // the root's row and slot
     }
 }
@@ -99,12 +105,61 @@ __device__ __forceinline__ void wideCheck(const WideBuild& b, int tid, int threa
     if (bad) atomicAdd(&b.c->bad, bad);
 }
 
-// A table has n leaves, so one that holds every triangle holds each of them once.
+__device__ __forceinline__ uint32_t loadStat(const uint32_t* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The wave's largest value into *p, all 64 lanes together.
+__device__ __forceinline__ void waveMax(uint32_t* p, uint32_t v)
+{
+    for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o));
+    if ((threadIdx.x & 63) == 0 && v > loadStat(p)) atomicMax(p, v);
+}
+// A large triangle's plane: its slot in the open-addressed table, claimed where it is new.
+__device__ __forceinline__ void notePlane(WideStats* st, uint32_t key, uint32_t sine)
+{
+    if (key != 0) {
+        const uint32_t home = (key * 2654435761u) >> 26;
+        for (int i = 0; i < kWidePlaneSlots; i++) {
+            const uint32_t at = (home + i) % kWidePlaneSlots;
+            uint32_t have = loadStat(&st->key[at]);
+            if (have == 0) {
+                have = atomicCAS(&st->key[at], 0u, key);
+                have = have == 0 ? key : have;
+            }
+            if (have == key) {
+                if (sine < loadStat(&st->sine[at])) atomicMin(&st->sine[at], sine);
+                return;
+            }
+        }
+    }
+    if (loadStat(&st->overflow) == 0) atomicMax(&st->overflow, 1u);
+}
+
+// Every triangle is a leaf of every table (which has n leaves, so it holds each of them
+// once), and what it is to the error bound of zgl_wide.h.
 __device__ __forceinline__ void wideTris(const WideBuild& b, int tid, int threads)
 {
+    const WideScale sc = wideScale(b.rows, b.rows + 3);
     int bad = 0;
-    for (int64_t g = tid; g < (int64_t)6 * b.n; g += threads)
-        if (b.rowOf[g] < 0) bad++;
+    uint32_t x = 0, diagonal = 0, edge = 0;
+    for (int64_t g = tid; g < b.n; g += threads) {
+        for (int t = 0; t < 6; t++)
+            if (b.rowOf[g * 6 + t] < 0) bad++;
+        const WideTriClass c = wideClassify(b.tris + g * 12, sc.bound);
+        if (c.kind == kWideTriBad) bad++;
+        if (c.kind == kWideTriSmall) {
+            x = max(x, fbits(c.x));
+            diagonal = max(diagonal, fbits(c.diagonal));
+        }
+        if (c.kind == kWideTriLarge) {
+            edge = max(edge, fbits(c.edge));
+            notePlane(&b.c->stats, c.key, fbits(c.sine));
+        }
+    }
+    waveMax(&b.c->stats.x, x);
+    waveMax(&b.c->stats.diagonal, diagonal);
+    waveMax(&b.c->stats.edge, edge);
     if (bad) atomicAdd(&b.c->bad, bad);
 }
 
@@ -233,9 +288,10 @@ int64_t wideCapacity(int64_t n) { return n + (2 * n) / 3 + 16; }
 size_t wideWorkBytes(int64_t n) { return align256(sizeof(WideCounters)) + 2 * align256((size_t)n * 8 + 8) + (size_t)n * 24; }
 
 hipError_t buildWide(const float4* rows, const float4* tris, int64_t nTri, void* work, uint4* slots, hipStream_t st,
-                     WideScale& scale)
+                     WideScale& scale, WideMargins& margins)
 {
     scale = WideScale{0.0f, 0.0f, 1.0f, false};
+    margins = WideMargins{};
     const int n = (int)nTri, S = 2 * n - 1;
     const int64_t capacity = wideCapacity(nTri);
     if (capacity > (int64_t)kWideSlotMask) return hipSuccess;
@@ -281,6 +337,7 @@ hipError_t buildWide(const float4* rows, const float4* tris, int64_t nTri, void*
         if (host.bad || host.slots > capacity) return hipSuccess;
         if (host.count[level] == 0) {
             scale = wideScale(host.root, host.root + 3);
+            margins = wideMargins(host.stats, scale);
             return hipSuccess;
         }
     }
