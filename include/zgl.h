@@ -109,6 +109,8 @@ typedef struct zgl_scene_buffers {
     int32_t sampler;              /* 0 independent, 1 Sobol (scene->sampler) */
 } zgl_scene_buffers;
 
+/* A refused scene leaves the context's as it was, but for one that the device build refuses
+ * (non-finite vertices) or that finds no memory: then there is none until the next upload. */
 zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* scene);
 
 /* Camera uniforms (src/integrator/NaivePath.cpp:49-60). mat_inv is column-major. */

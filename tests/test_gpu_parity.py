@@ -99,6 +99,27 @@ def test_upload_rejects_nonfinite_bounds(ctx, c1):
     ctx.upload(c1)
 
 
+def test_upload_that_fails_on_the_device_leaves_no_scene(ctx, c1):
+    """The device build refuses a vertex after the context's buffers were replaced: rays and
+    passes are refused until a scene is uploaded again, not run over the mixture."""
+    import copy
+    good = scene.pack(scene.config1(), bvh="device")
+    bad = copy.copy(good)
+    bad.vertices = good.vertices.copy()
+    bad.vertices[4, 1] = np.nan
+    ctx.upload(good)
+    with pytest.raises(_lib.ZglError) as e:
+        ctx.upload(bad)
+    assert e.value.status == _lib.ZGL_E_INVALID
+    rays = scene.ray_batch(1000, seed=5)
+    for call in (lambda: ctx.trace_closest(rays), lambda: ctx.render(_lib.INTEGRATOR_NAIVE, 0, 1, 1, 3)):
+        with pytest.raises(_lib.ZglError) as e:
+            call()
+        assert e.value.status == _lib.ZGL_E_STATE
+    ctx.upload(c1)
+    assert np.array_equal(ctx.trace_closest(rays)[0], orc.trace_closest(c1, rays)[0])
+
+
 def test_closest_hit_counters_match_oracle(ctx, c1):
     ctx.upload(c1)
     rays = scene.ray_batch(100_000, seed=5)

@@ -462,6 +462,9 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
                 std::memcpy(o + 6, &r[1], 4);
                 std::memcpy(o + 7, &miss, 4);
             }
+        // from here on buffers that the context's scene points to are replaced: an upload that
+        // fails leaves the context without a scene
+        ctx->hasScene = false;
         if (!deviceBvh) ctx->upload(ctx->rows, rows.data(), rows.size() * 4, "rows");
         ctx->upload(ctx->indices, sb->indices, (size_t)nT * 12, "indices");
         ctx->upload(ctx->vertices, sb->vertices, (size_t)nV * 12, "vertices");
