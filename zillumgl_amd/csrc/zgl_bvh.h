@@ -33,6 +33,8 @@ public:
     int build(const float* dVerts, int64_t nV, const uint32_t* dIdx, int64_t nT, int subtree, float* dBounds,
               int32_t* dHit, void* dRows, hipStream_t st, std::string& err);
     void release();
+    // The work memory of the last build for another use until the next (null: less than `bytes`).
+    void* work(size_t bytes) const { return workBytes_ >= bytes ? work_ : nullptr; }
     DeviceBvhStats stats;
 
 private:

@@ -157,8 +157,7 @@ struct zgl_context {
     // differentiable mode: evaluation point, adjoint input and outputs
     DevBuf evalMat, evalEnv, dFrame, dMat, dEnv;
     DevBuf bvhBounds;  // node bounds of a device-built MTBVH
-    DevBuf envRaw;     // upload staging of the environment map
-    DevBuf wide;       // 4-wide tree, then its builder's work memory
+    DevBuf wide;       // 4-wide tree
     DevBuf gqQueues, gqCounts;  // global-queue path tracer
     int gqBlocksPerCU = 0;
     DevBuf wfWork;    // wavefront schedule of the naive tracer
@@ -192,7 +191,7 @@ struct zgl_context {
                          &lightPower, &lightAlias, &lightProb, &env, &envAlias, &envProb, &noise, &sobolM,
                          &sobolTab, &frame, &film, &counters, &scratchRays, &scratchOut, &workCounter,
                          &evalMat, &evalEnv, &dFrame, &dMat, &dEnv, &bvhBounds, &gqQueues, &gqCounts, &wfWork,
-                         &naiveRes, &hitLog, &refSum, &tex, &texScale, &texRaw, &envRaw, &wide};
+                         &naiveRes, &hitLog, &refSum, &tex, &texScale, &texRaw, &wide};
         for (DevBuf* b : all) b->release();
         bvh.release();
     }
@@ -465,6 +464,9 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
         // from here on buffers that the context's scene points to are replaced: an upload that
         // fails leaves the context without a scene
         ctx->hasScene = false;
+        // a wide tree too small for this scene makes room for the buffers first
+        const size_t wideBytes = (size_t)wideCapacity(nT) * 64;
+        if (ctx->wide.bytes < wideBytes) ctx->wide.release();
         if (!deviceBvh) ctx->upload(ctx->rows, rows.data(), rows.size() * 4, "rows");
         ctx->upload(ctx->indices, sb->indices, (size_t)nT * 12, "indices");
         ctx->upload(ctx->vertices, sb->vertices, (size_t)nV * 12, "vertices");
@@ -482,23 +484,6 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
                                           ctx->stream, msg);
             if (rc) throw ZglError{rc == 1 ? ZGL_E_INVALID : (rc == 3 ? ZGL_E_OOM : ZGL_E_HIP), msg};
         }
-        // a device too full for the wide tree renders over the rows, with the same results
-        WideScale wideScale{};
-        WideMargins wideMargins{};
-        const size_t wideBytes = (size_t)wideCapacity(nT) * 64;
-        bool wideFits = true;
-        try {
-            ctx->ensure(ctx->wide, wideBytes + wideWorkBytes(nT), "wide tree");
-        } catch (const ZglError& e) {
-            if (e.code != ZGL_E_OOM) throw;
-            (void)hipGetLastError();
-            wideFits = false;
-        }
-        if (wideFits)
-            hipCheck(buildWide((const float4*)ctx->rows.p, (const float4*)ctx->tris.p, nT,
-                               (char*)ctx->wide.p + wideBytes, (uint4*)ctx->wide.p, ctx->stream, wideScale,
-                               wideMargins),
-                     "wide tree build");
         ctx->upload(ctx->normals, sb->normals, (size_t)nV * 12, "normals");
         ctx->upload(ctx->texcoords, sb->texcoords, (size_t)sb->n_texcoords * 8, "texcoords");
         ctx->upload(ctx->matTex, sb->mat_tex_indices, (size_t)sb->obj_prim_count * 4, "matTexIndices");
@@ -507,9 +492,12 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
         ctx->upload(ctx->lightPower, sb->light_power, (size_t)nL * 12, "lightPower");
         ctx->upload(ctx->lightAlias, sb->light_alias, (size_t)nL * 4, "lightAlias");
         ctx->upload(ctx->lightProb, sb->light_prob, (size_t)nL * 4, "lightProb");
-        ctx->upload(ctx->envRaw, sb->env_rgb16f, (size_t)w * h * 6, "env");
+        // the texels as they come go where the evaluation point's will be
+        ctx->ensure(ctx->evalEnv, (size_t)w * h * 16, "eval env");
+        hipCheck(hipMemcpyAsync(ctx->evalEnv.p, sb->env_rgb16f, (size_t)w * h * 6, hipMemcpyHostToDevice, ctx->stream),
+                 "env");
         ctx->ensure(ctx->env, (size_t)w * h * 8, "env");
-        hipCheck(launchPackEnv((const uint16_t*)ctx->envRaw.p, (ushort4*)ctx->env.p, (int64_t)w * h, ctx->stream), "env");
+        hipCheck(launchPackEnv((const uint16_t*)ctx->evalEnv.p, (ushort4*)ctx->env.p, (int64_t)w * h, ctx->stream), "env");
         ctx->upload(ctx->envAlias, sb->env_alias, (size_t)(w + 1) * h * 4, "envAlias");
         ctx->upload(ctx->envProb, sb->env_prob, (size_t)(w + 1) * h * 4, "envProb");
         hipCheck(hipStreamSynchronize(ctx->stream), "scene upload");
@@ -517,10 +505,7 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
         DevScene& s = ctx->scene;
         s.rows = (const float4*)ctx->rows.p;
         s.tris = (const float4*)ctx->tris.p;
-        s.wide = wideScale.ok ? (const uint4*)ctx->wide.p : nullptr;
-        s.wideUnit = wideScale.unit;
-        s.wideBound = wideScale.bound;
-        s.wideMargins = wideMargins;
+        s.wide = nullptr;
         s.indices = (const int32_t*)ctx->indices.p;
         s.vertices = (const float*)ctx->vertices.p;
         s.normals = (const float*)ctx->normals.p;
@@ -552,8 +537,30 @@ zgl_status zgl_upload_scene(zgl_context* ctx, const zgl_scene_buffers* sb)
         // evaluation point of the differentiable mode: the uploaded values
         ctx->hostMaterials.assign(sb->materials, sb->materials + (size_t)sb->n_materials * 16);
         ctx->upload(ctx->evalMat, sb->materials, (size_t)sb->n_materials * 64, "eval materials");
-        ctx->ensure(ctx->evalEnv, (size_t)w * h * 16, "eval env");
         hipCheck(launchEnvExpand(s.env, (float4*)ctx->evalEnv.p, (int64_t)w * h, ctx->stream), "eval env");
+        // the wide tree last, so that it takes no memory from the rest: a device too full for it
+        // renders over the rows, with the same results.  Its builder works in the MTBVH build's
+        // memory, or in some of its own that is given back.
+        struct Temporary : DevBuf { ~Temporary() { release(); } } own;
+        WideScale wideScale{};
+        s.wideMargins = WideMargins{};
+        void* work = nullptr;
+        try {
+            ctx->ensure(ctx->wide, wideBytes, "wide tree");
+            work = deviceBvh ? ctx->bvh.work(wideWorkBytes(nT)) : nullptr;
+            if (!work) ctx->ensure(own, wideWorkBytes(nT), "wide tree");
+            if (!work) work = own.p;
+        } catch (const ZglError& e) {
+            if (e.code != ZGL_E_OOM) throw;
+            (void)hipGetLastError();
+            ctx->wide.release();
+        }
+        if (work)
+            hipCheck(buildWide(s.rows, s.tris, nT, work, (uint4*)ctx->wide.p, ctx->stream, wideScale, s.wideMargins),
+                     "wide tree build");
+        s.wide = wideScale.ok ? (const uint4*)ctx->wide.p : nullptr;
+        s.wideUnit = wideScale.unit;
+        s.wideBound = wideScale.bound;
         hipCheck(hipStreamSynchronize(ctx->stream), "scene upload");
         ctx->hasScene = true;
     });
