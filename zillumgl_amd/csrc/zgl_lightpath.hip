@@ -40,7 +40,7 @@ enum : int {
     kDone,
 };
 
-constexpr int kNodesPerRound = 3;  // as the naive tracer's
+constexpr int kNodesPerRound = 2;  // as the naive tracer's
 
 __global__ void k_reset_light_counter(int* c)
 {

@@ -36,10 +36,11 @@ enum : int {
 };
 
 // Nodes of the wide tree each walking lane advances per round of the walking loop (one
-// triangle test and one ballot per round).  1 / 2 / 3 / 4: 124.0 / 116.5 / 114.8 / 114.9 ms
-// on the headline launch, 24.5 / 23.0 / 22.3 / 21.9 ms on ten batched scenes, 2.78 / 2.69 /
-// 2.70 / 2.80 ms on the material scene.
-constexpr int kNodesPerRound = 3;
+// triangle test and one ballot per round).  2 / 3 / 4: 100.4 / 100.8 / 103.1 ms on the
+// headline launch, 16.7 / 16.6 / 17.5 ms on ten batched scenes, 2.39 / 2.50 / 2.55 ms on the
+// material scene; 2 / 3: 901 / 969 us for a 720p pass, 123 / 134 us for a 256 x 256 pass of
+// the Cornell box, 12.0 / 12.5 ms in the triple tracer.
+constexpr int kNodesPerRound = 2;
 
 // The pixel and the pass of a work unit: units are in (8x8 tile, pass, pixel of the tile)
 // order, tiles row by row.
