@@ -1,7 +1,10 @@
-"""Ray batches over the device-built 4-wide tree against the counting kernel, which walks the
-reference's rows: the same primitives and distance bits; any-hits against the host build of
-the rows' walk.  Scenes the wide tree refuses (a caller's boxes that are not the triangles'
-own, trees deeper than its builder goes) render over the rows."""
+"""Walks over the device-built 4-wide tree against the counting kernels, which walk the
+reference's rows: ray batches with the same primitives and distance bits, any-hits against
+the host build of the rows' walk, frames bit for bit.  Batches on scenes of fewer than 2,048
+triangles walk the rows whatever the tree, so the batch tests' scenes are padded past that;
+the frames are of the small scenes themselves, whose trees one workgroup or a few levels
+build.  Scenes that the builder refuses (a caller's boxes that are not the triangles' own,
+"identical", whose tree is deeper than it goes) give the rows' results too."""
 import numpy as np
 import pytest
 
@@ -37,7 +40,27 @@ def _compare(probe, ps, n, r=None):
 
 @pytest.mark.parametrize("name", sorted(SCENES))
 def test_batches_equal_the_rows(probe, name):
-    _compare(probe, scene.pack(SCENES[name]), 20000)
+    ps = scene.pack(wide_rays.padded(SCENES[name]))
+    assert ps.indices.shape[0] >= 2048
+    _compare(probe, ps, 20000)
+
+
+@pytest.mark.parametrize("name", ["cornell", "materials", "caustics", "tessellated", "soup1", "soup2", "soup3", "soup4",
+                                  "soup5", "soup300", "duplicates", "identical", "slivers"])
+def test_frames_equal_the_rows(name):
+    ps = scene.pack(SCENES[name], bvh="device")
+    ctx = render.Context(0)
+    try:
+        frames = []
+        for count in (False, True):
+            ctx.upload(ps)
+            ctx.clear()
+            ctx.render(0, 0, 16, 1, 5, count_bytes=count)
+            frames.append(ctx.read_frame())
+        assert np.isfinite(frames[1]).all()
+        np.testing.assert_array_equal(frames[0].view(np.int32), frames[1].view(np.int32))
+    finally:
+        ctx.close()
 
 
 @pytest.mark.parametrize("n", [1000, 100003])
