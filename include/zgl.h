@@ -173,12 +173,11 @@ typedef struct zgl_pass_params {
     int32_t loops_per_pass;       /* triple: LPTLoopsPerPass */
     int32_t count_bytes;          /* accumulate algorithmic-byte counters (slower) */
     int32_t regen_threshold;      /* naive, light, triple (persistent kernels): lanes of a wave64
-                                     still walking the MTBVH when the wave stops to shade and
+                                     still walking when the wave stops to shade and
                                      reissue rays (1..63).  0 = default: for the naive tracer and
-                                     the triple tracer's camera pass 1 + (m - 1) f, where m =
-                                     0.7 log2 n - 2.5 clamped to 1..16 for n triangles and f =
-                                     0.2 + u / 48, at most 1, for u samples per resident lane;
-                                     1 for light paths.  Frames do not depend on it. */
+                                     the triple tracer's camera pass 1 + 11 f, where f = 0.2 +
+                                     u / 48, at most 1, for u samples per resident lane; 2 for
+                                     light paths.  Frames do not depend on it. */
 } zgl_pass_params;
 /* ZGL_INTEGRATOR_NAIVE keeps each sample's value (16 bytes) in a context-owned buffer of
  * at most 4 GiB and adds them to the frame in pass order; calls with more passes than fit

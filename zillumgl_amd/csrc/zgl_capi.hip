@@ -20,28 +20,28 @@ using namespace zgl;
 
 // zgl_render's default for it (regen_threshold 0): how many lanes of a wave may still be
 // walking when the wave stops to shade.  Frames do not depend on it.  Shading early keeps
-// lanes walking and shades with few lanes; it pays with long walks, and with enough units
-// for every lane that a wave which shades can refill its idle lanes: a launch of a few
-// units per lane ends sooner the fewer shading steps its waves make.
+// lanes walking and shades with few lanes; it pays with enough units for every lane that
+// a wave which shades can refill its idle lanes: a launch of a few units per lane ends
+// sooner the fewer shading steps its waves make.
 // Sweeps on one MI355X (1024 x 1024, depth 8; ms at the best value, then the time at
 // 4 / 12 / 24 over the best):
-//   16 passes (64 units per lane)          1 pass (4 units per lane)
-//   36 triangles      16.6 at 1: 1.04 1.16 1.43     1.22 at 1:  1.10 1.36 1.73
-//   852               17.8 at 3: 1.00 1.10 1.39     1.70 at 2:  1.04 1.26 1.59
-//   9,828             19.0 at 6: 1.01 1.05 1.32     1.89 at 2:  1.03 1.20 1.51
-//   99,146            22.9 at 12: 1.07 1.00 1.15    2.47 at 4:  1.00 1.11 1.33
-//   1,306,146         31.8 at 12: 1.17 1.00 1.04    4.18 at 12: 1.01 1.00 1.16
+//   16 passes (64 units per lane)           1 pass (4 units per lane)
+//   36 triangles      13.8 at 12: 1.05 1.00 1.08     1.28 at 2: 1.01 1.09 1.26
+//   852               18.4 at 12: 1.03 1.00 1.01     1.67 at 3: 1.01 1.05 1.20
+//   9,828             20.0 at 8: 1.03 1.00 1.01      1.89 at 4: 1.00 1.05 1.22
+//   99,146            25.1 at 12: 1.06 1.00 1.01     2.47 at 3: 1.05 1.05 1.17
+//   1,306,146         34.9 at 16: 1.11 1.00 1.00     4.07 at 6: 1.03 1.05 1.10
 //   819,400 (headline, 1080p, 127 and 8 units per lane)
-//                     27.7 at 12: 1.03 1.00 1.08    2.88 at 4:  1.00 1.12 1.34
-// The rule below is within 4% of the best in all of them and in the triple tracer's
-// camera pass; light paths, short everywhere, were fastest at 1 or 2 at every size.
-static int defaultThreshold(int bvhSize, double unitsPerLane)
+//                     28.4 at 12: 1.05 1.00 1.03     3.57 at 6: 1.03 1.05 1.21
+// With rounds of two nodes the triangle count does not matter any more.  The rule below is
+// within 3% of the best in all of them, at 0.25, 2 and 32 units per lane (best 3, 4 and 12)
+// and in the triple tracer's camera pass (12 at 64 units per lane); light paths took 2.64 /
+// 2.52 / 2.51 ms at 1 / 2 / 4 with 16 passes and 0.97 / 0.96 / 0.98 with 2.
+static int defaultThreshold(double unitsPerLane)
 {
-    const double l = std::log2((double)std::max(2, (bvhSize + 1) / 2));
-    const double most = std::min(16.0, std::max(1.0, 0.7 * l - 2.5));
-    return (int)std::lround(1.0 + (most - 1.0) * std::min(1.0, 0.2 + unitsPerLane / 48.0));
+    return (int)std::lround(1.0 + 11.0 * std::min(1.0, 0.2 + unitsPerLane / 48.0));
 }
-constexpr int kLightPathThreshold = 1;
+constexpr int kLightPathThreshold = 2;
 // Largest sample-value plus traversal-log buffer of one chunk of the differentiable mode's passes.
 constexpr size_t kAdjointLogBytes = (size_t)8 << 30;
 // Largest total of a batch's per-sample value buffers.
@@ -788,7 +788,7 @@ static int naiveThreshold(const zgl_context* ctx, int requested, int nPasses, in
 {
     if (requested > 0) return requested;
     const double lanes = 256.0 * std::max(1, ctx->numCUs * blocksPerCU);
-    return defaultThreshold(ctx->scene.bvhSize, (double)ctx->filmW * ctx->filmH * nPasses / lanes);
+    return defaultThreshold((double)ctx->filmW * ctx->filmH * nPasses / lanes);
 }
 
 // Validates a pass request and builds the per-launch scene view and parameters.
@@ -1278,7 +1278,7 @@ static void batchUpload(zgl_batch* b)
         const zgl_pass_params* p = &b->params[i];
         BatchScene& it = b->host[k];
         it.s = ctx->scene;
-        it.threshold = b->threshold > 0 ? b->threshold : defaultThreshold(it.s.bvhSize, unitsPerLane);
+        it.threshold = b->threshold > 0 ? b->threshold : defaultThreshold(unitsPerLane);
         it.s.sobolTab = (const uint32_t*)b->sobolTab.p;
         it.s.sobolTabFirst = b->sobolFirst;
         it.s.sobolTabCount = b->sobolCount;
