@@ -1,6 +1,6 @@
 """Walks over the device-built 4-wide tree against the counting kernels, which walk the
 reference's rows: ray batches with the same primitives and distance bits, any-hits against
-the host build of the rows' walk, frames bit for bit.  Batches on scenes of fewer than 2,048
+the host build of the rows' walk, frames bit for bit.  Batches on scenes of fewer than 1,024
 triangles walk the rows whatever the tree, so the batch tests' scenes are padded past that;
 the frames are of the small scenes themselves, whose trees one workgroup or a few levels
 build.  Scenes that the builder refuses (a caller's boxes that are not the triangles' own,
@@ -65,7 +65,7 @@ def test_frames_equal_the_rows(name):
 
 @pytest.mark.parametrize("n", [1000, 100003])
 def test_batch_sizes(probe, n):
-    ps = scene.pack(scene.config5(32, 32, n=20, env_size=(8, 4)))  # above the rule's 2,048 triangles
+    ps = scene.pack(scene.config5(32, 32, n=20, env_size=(8, 4)))  # above the rule's 1,024 triangles
     _compare(probe, ps, n)
 
 

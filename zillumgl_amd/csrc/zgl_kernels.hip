@@ -591,10 +591,11 @@ hipError_t launchFilmToFrame(const float* film, float4* frame, int w, int h, hip
     return hipGetLastError();
 }
 // A batch on a scene of fewer triangles walks the rows.  Measured on tessellated Cornell
-// boxes, 10^6 incoherent rays, over the rows / over the wide tree: 36 triangles 90 / 116
-// us, 546 157 / 171, 1,226 173 / 179, 2,756 194 / 181.  A ray's few rows cost as little
-// there, and the kernel without walk stacks keeps twice the waves on a compute unit.
-constexpr int kBatchRowsBelow = 2048;
+// boxes, 10^6 incoherent rays, over the rows / over the wide tree: 36 triangles 84 / 117
+// us, 546 171 / 183, 1,226 213 / 182, 1,668 206 / 193, 2,178 272 / 193, 5,748 288 / 209.  A
+// ray's few rows cost as little there, and the kernel without walk stacks keeps twice the
+// waves on a compute unit.
+constexpr int kBatchRowsBelow = 1024;
 static inline bool batchOverRows(const DevScene& s) { return !s.wide || s.nTriangles < kBatchRowsBelow; }
 
 hipError_t launchTraceClosest(const DevScene& s, const float* rays, int64_t n, int32_t* prim, float* t,
