@@ -7,8 +7,9 @@ Sobol sampler, NEE on, Russian roulette off.  One step = one 64-spp frame (64
 progressive passes in one launch of the path-tracing kernel) with the scene already
 resident in HBM.  Metric: Msamples/s = 1920 * 1080 * 64 / t_step / 1e6.
 
-Also reported: the HBM roofline of the path-tracing kernel (the measured L2-to-fabric
-bytes of a launch over the kernel's average duration from HIP events on its stream),
+Also reported: the roofline that bounds the path-tracing kernel (VALU issue, from the
+committed counter profile), its HBM side (the measured L2-to-fabric bytes of a launch
+over the kernel's average duration from HIP events on its stream),
 the algorithmic bytes of the reference's walk (counted by the kernel's counting variant
 in the reference's data layout: 36 B per MTBVH row visited, 48 B per leaf triangle test,
 108 B per surface interaction, ...; the timed kernel walks a 4-wide tree and reads a
@@ -27,6 +28,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+# vector instructions a second: 256 CUs x 4 SIMDs x 2.4 GHz, four cycles for 64 lanes
+VALU_PEAK_GINST = 614.4
 
 
 class Hip:
@@ -478,17 +481,22 @@ def main():
         traffic = profile_value(f"naive_{args.workload}_traffic.md", "hbm_bytes_per_launch")
         lanes = profile_value(f"naive_{args.workload}_valu.md", "active_lanes_per_valu")
         busy = profile_value(f"naive_{args.workload}_valu.md", "valu_issue_busy")
+        issue = min(1.0, busy) if busy else None  # a ratio above 1: some take less than four cycles
         fabric = traffic / avg_s / 1e9 if traffic else None
-        # achieved/frac: the measured L2-to-fabric traffic.  The counted bytes are those of
-        # the reference's row walk, of which the 4-wide walk reads a part: over the time
-        # they are no bandwidth, only a figure to compare with other kernels of that walk.
-        # The measured limiter (VALU issue, lane use) is from the counter profile.
-        roofline = {"bound": "hbm", "achieved": round(fabric, 1) if fabric else None, "peak": HBM_PEAK_GBS,
-                    "unit": "GB/s", "frac": round(fabric / HBM_PEAK_GBS, 4) if fabric else None, "traffic": traffic,
-                    "achieved_is": "measured L2-to-fabric bytes per launch / event-timed launch",
+        # achieved/frac: the share of the SIMDs' cycles that issue a vector instruction, from
+        # the counter profile.  hbm: the measured L2-to-fabric traffic.  The counted bytes are
+        # those of the reference's row walk, of which the 4-wide walk reads a part: over the
+        # time they are no bandwidth, only a figure to compare with other kernels of that walk.
+        roofline = {"bound": "valu", "achieved": round(issue * VALU_PEAK_GINST, 1) if issue else None,
+                    "peak": VALU_PEAK_GINST, "unit": "G wave64 VALU instructions/s", "frac": issue,
+                    "achieved_is": "issue cycles of profiles/naive_c2_valu.md's launch",
+                    "hbm": {"achieved": round(fabric, 1) if fabric else None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                            "frac": round(fabric / HBM_PEAK_GBS, 4) if fabric else None,
+                            "achieved_is": "measured L2-to-fabric bytes per launch / event-timed launch"},
+                    "traffic": traffic,
                     "reference_walk_GBps": round(achieved, 1),
-                    "limiter": (f"VALU issue ({busy:.0%} busy, {lanes:.1f} of 64 lanes active per VALU instruction)"
-                                if lanes and busy else None),
+                    "limiter": (f"VALU issue ({issue:.0%} busy, {lanes:.1f} of 64 lanes active per VALU instruction)"
+                                if lanes and issue else None),
                     "algorithmic_bytes_per_launch": algo_bytes,
                     "bytes_per_sample": round(algo_bytes / samples, 1),
                     "rows_per_traversal": round(float(cnt[1]) / max(float(cnt[3]), 1.0), 2),

@@ -455,7 +455,7 @@ __global__ __launch_bounds__(256, 4) void k_naive_batch(const BatchScene* __rest
 // ---------------------------------------------------------------------------
 // Triple path tracer, camera pass (triple_path_pass_pt.glsl:44-195) on the same
 // persistent schedule: one sample per (8x8 tile, pass) unit, XCD regions, walks advanced
-// a few rows per ballot round with lanes shading and reissuing rays once no more than
+// a few nodes per ballot round with lanes shading and reissuing rays once no more than
 // `threshold` are still walking.  The shading steps are tripleCameraTrace's, in its order
 // of operations and random-number use; the s=1 term is evaluated before its visibility
 // walk and added if the walk finds no occluder.  Each sample's value goes to

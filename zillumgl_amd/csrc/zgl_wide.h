@@ -1,9 +1,9 @@
 // zgl_wide.h -- closest-hit and any-hit walks over a 4-wide tree, with results equal to
 // the reference's MTBVH walk (intersection.glsl:367-427) bit for bit; host and device.
 //
-// What bounds the reference's walk is its rows: on the 819,400-triangle scene a ray visits
-// 47 of them, each a dependent 32-byte load and an exact box test of about 45 vector
-// instructions.  Only two things of that walk reach its result: which triangles' own
+// What bounds the reference's walk is its rows: on the 819,400-triangle scene a walk visits
+// 56 of them on average, each a dependent 32-byte load and an exact box test of about 45
+// vector instructions.  Only two things of that walk reach its result: which triangles' own
 // boxes and all their ancestors' boxes pass the box test, and the order in which hits
 // shrink the distance.  The walk here visits a collapsed tree of the same leaves (four
 // children per 64-byte node, FP16 planes rounded outwards and padded, nearest child
@@ -67,17 +67,19 @@
 // wideMargins makes from the scene's largest X, diagonal and edge the limit (rel, slack)
 // up to which a walk has to keep subtrees.
 //
-// Measured: 47 rows become 13 nodes and 3 triangles a ray on the headline scene.  A node
-// step is about 110 vector instructions for four boxes (fma_mix reads the FP16 planes in
-// place) against 45 for one row.
+// Measured: the headline launch's walks visit 15 nodes and 3 triangles each (as it was counted
+// with subtrees dropped at 1.001 t: 14 and 2.8); 64 passes at 1080p take 100 ms, 169 over the
+// rows, 95 with subtrees dropped at 1.001 t.  A node step is about 110 vector instructions
+// for four boxes (fma_mix reads the FP16 planes in place) against 45 for one row.
 //
 // Rays the argument does not cover take the reference's rows from the start: nearly
 // axis-parallel ones (RayPre::mode != 0), components below 1e-6, not finite, from far
 // outside the scene, or with a direction longer than 1 or shorter (any-hits: than 0.5).
 // For a ray with one component below 1e-6 the reference's test drops that axis' slab, and
-// its walk visits every box of a slice through the scene (15 ms for one ray on a
-// 205,000-triangle scene).  Boxes further from the ray on that axis than a hit can lie
-// beside its triangle are left out of that walk (rowHit).
+// its walk visits every box of a slice through the scene (one ray in a 1280 x 720 pass over
+// 205,000 triangles held up the launch to 15 ms).  Boxes further from the ray on that axis
+// than a hit can lie beside its triangle are left out of that walk (rowHit), which leaves
+// about 120 rows: the pass takes 1.6 ms alone and 0.9 among others.
 #pragma once
 
 #include "zgl_box.h"
