@@ -148,8 +148,9 @@ extern "C" void probe_wide_trace(const float* rays, int64_t n, const float* tmax
 }
 
 // The margins of the built tree.
-extern "C" void probe_wide_margins(float out[5])
+extern "C" void probe_wide_margins(float out[6])
 {
-    const float v[5] = {g.margins.rel, g.margins.slack, g.margins.grow, g.margins.growRel, g.margins.reach};
+    const float v[6] = {g.margins.rel,     g.margins.slack, g.margins.grow,
+                        g.margins.growRel, g.margins.reach, (float)g.margins.nPlanes};
     std::memcpy(out, v, sizeof(v));
 }

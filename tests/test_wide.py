@@ -49,6 +49,21 @@ def test_rays_nearly_in_a_triangles_plane(probe, name, scale, turned):
         np.testing.assert_array_equal(occ >= 0, ref >= 0)
 
 
+@pytest.mark.parametrize("name,scale,planes,drops", [("cornell", 1, 4, True), ("cornell", 100, 4, True),
+                                                     ("spheres", 1, 0, True), ("spheres", 100, 0, False),
+                                                     ("caustics", 1, 4, True), ("caustics", 1000, 0, False)])
+def test_margins_of_a_scene(probe, name, scale, planes, drops):
+    """The large triangles' planes where they are few; where they are many nothing is dropped and
+    no box is left out beside a ray, whatever the distance."""
+    ps = scene.pack(wide_rays.scaled(SCENES[name], scale))
+    assert probe.build(ps) > 0
+    rel, slack, grow, grow_rel, reach, n = probe.margins()
+    bound = float(np.abs(ps.vertices).max())
+    assert n == planes
+    assert 1.0009 < rel < 1.2 if drops else slack == np.inf
+    assert 0 < slack < 0.2 * bound if drops else grow >= 8 * bound
+
+
 def _hits(tri, o, d):
     """intersectTriangle (src/shader/intersection.glsl:63-109) in FP32, operation by operation:
     the mask of hits, t and |det|."""

@@ -27,6 +27,12 @@ class Probe:
                                          C.c_int64(ps.indices.shape[0]), p(ps.bounds, C.c_float),
                                          p(ps.hit_table, C.c_int32))
 
+    def margins(self):
+        """rel, slack, grow, growRel, reach and the number of planes of the built tree."""
+        out = (C.c_float * 6)()
+        self.lib.probe_wide_margins(out)
+        return list(out)
+
     def trace(self, rays, tmax=None, rows_only=False):
         """Closest hits (prim, t), or any-hits with tmax: prim >= 0 where occluded; and the
         walk's statistics (see the source)."""

@@ -280,7 +280,7 @@ inline WideMargins wideMargins(const WideStats& st, const WideScale& sc)
         m.nPlanes = 0;
         m.rel = 1.0f;
         m.slack = __builtin_inff();
-        m.growRel = 1e9f;  // past the scene's end
+        m.grow = 8.0f * sc.bound;  // past the scene's end, whatever the distance
         return m;
     }
     double rel = 1.03 * c / (1.0 - c), abs = 1.03 * diagonal / (1.0 - c);
